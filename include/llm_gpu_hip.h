@@ -256,7 +256,10 @@ int lgh_probe_read_dev(lgh_ctx *ctx, const void *src_dev, size_t bytes, int per_
  * OutputHead::apply (weights.rs:186-192): per token, y[n] = W[n,k] @ x[k]
  * with per-block ActQ8 activations.  Assign mode only, as in the reference.
  * Any K and any number of tokens (rows past 32768 elements are summed in
- * K ranges of 32768, added in f32). */
+ * K ranges of 32768, added in f32).  Several tokens of a large matrix share
+ * one pass over the weights per 64 tokens, on an activation image in the
+ * context's workspace (a captured call that would have to grow it reads the
+ * weights once per token instead). */
 int lgh_q8_gemv(lgh_ctx *ctx, const lgh_q8 *w, const float *x, float *y, size_t tokens);
 int lgh_q8_gemv_dev(lgh_ctx *ctx, const lgh_q8 *w, const float *x_dev, float *y_dev,
                     size_t tokens);
@@ -264,7 +267,8 @@ int lgh_q8_gemv_dev(lgh_ctx *ctx, const lgh_q8 *w, const float *x_dev, float *y_
 /* The final rms_norm of a decode or prefill step followed by the Q8_0 output
  * head (crates/llm-engine/src/lfm2.rs:559-567, 496-504): per token,
  * y = W (rms_norm(hidden, norm_w, eps)), norm_w == NULL: y = W hidden -- the
- * norm in the GEMV's prologue, one launch.  (A Q4 head takes lgh_q4_norm_gemv
+ * norm in the GEMV's prologue (one launch), or in the launch that writes the
+ * activation image of several tokens.  (A Q4 head takes lgh_q4_norm_gemv
  * with one matrix.)  Results equal rms_norm followed by lgh_q8_gemv. */
 int lgh_q8_norm_gemv(lgh_ctx *ctx, const lgh_q8 *w, const float *norm_w, float eps, const float *hidden, float *y,
                      size_t tokens);

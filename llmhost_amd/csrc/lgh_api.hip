@@ -1083,6 +1083,50 @@ int lgh_probe_read_dev(lgh_ctx *ctx, const void *src_dev, size_t bytes, int per_
   return LGH_OK;
 }
 
+// Whether the context stream is being captured (growing a workspace fails then).
+static bool capturing(lgh_ctx *ctx) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(ctx->stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
+}
+
+// The Q8_0 product of `tokens` rows of x, rms_norm'd first when nw is not null.
+// Several tokens of a large matrix: up to 64 at a time, their activation image
+// (with the norm) and one pass over the weights.  Otherwise, and where
+// the image's workspace would have to grow under capture, the GEMV.
+static int q8_rows(lgh_ctx *ctx, const lgh_q8 *w, const float *x, const float *nw, float eps, float *y,
+                   size_t tokens) {
+  const size_t k = w->k, pq = (w->bpr + 3) / 4;
+  // Passes of up to 64 tokens, evenly filled in whole 16-token tiles.
+  const size_t passes = (tokens + 63) / 64, mt = ((tokens + passes - 1) / passes + 15) / 16, chunk = mt * 16;
+  Carve cv;
+  const size_t o_ci = cv.take(mt * pq * 2 * 1024), o_si = cv.take(mt * pq * 256);
+  if (lgh::q8_batch_wanted(w, tokens) && (cv.off <= ctx->ws_bytes || !capturing(ctx))) {
+    char *ws = nullptr;
+    if (int r = grow_ws(ctx).get(cv.off, &ws)) return r;
+    auto *ci = reinterpret_cast<uint8_t *>(ws + o_ci);
+    auto *si = reinterpret_cast<float *>(ws + o_si);
+    lgh::ActPrologue pro;
+    pro.nw = nw;
+    pro.eps = eps;
+    for (size_t t0 = 0; t0 < tokens; t0 += chunk) {
+      const size_t mc = std::min(chunk, tokens - t0);
+      LGH_HIP(ctx, lgh::launch_act_quant_mma(x + t0 * k, pro, mc, k, 0, ci, si, nullptr, ctx->stream,
+                                             lgh::MmaOrder::kPair));
+      LGH_HIP(ctx, lgh::launch_q8_mma(w, ci, si, y + t0 * w->n, mc, ctx->stream));
+    }
+    return LGH_OK;
+  }
+  if (nw && k > lgh::kQ8GemvMaxK) {  // rows longer than the prologue covers: rms_norm first
+    if (int r = ensure(ctx, &ctx->ffn, &ctx->ffn_bytes, tokens * k * sizeof(float))) return r;
+    float *nd = static_cast<float *>(ctx->ffn);
+    LGH_HIP(ctx, lgh::launch_rms_norm(x, nw, k, tokens, eps, nd, ctx->stream));
+    x = nd;
+    nw = nullptr;
+  }
+  LGH_HIP(ctx, lgh::launch_q8_gemv(w, x, y, tokens, nw, eps, ctx->stream));
+  return LGH_OK;
+}
+
 int lgh_q8_gemv_dev(lgh_ctx *ctx, const lgh_q8 *w, const float *x_dev, float *y_dev, size_t tokens) {
   if (!ctx) return LGH_ERR_INVALID_ARG;
   if (int r = check_mat(ctx, w)) return r;
@@ -1090,8 +1134,7 @@ int lgh_q8_gemv_dev(lgh_ctx *ctx, const lgh_q8 *w, const float *x_dev, float *y_
   if (!y_dev || (w->k && !x_dev)) return fail(ctx, LGH_ERR_INVALID_ARG, "null x/y");
   if (!aligned16(x_dev)) return fail(ctx, LGH_ERR_INVALID_ARG, "x must be 16-byte aligned");
   if (int r = set_device(ctx)) return r;
-  LGH_HIP(ctx, lgh::launch_q8_gemv(w, x_dev, y_dev, tokens, nullptr, 0.0f, ctx->stream));
-  return LGH_OK;
+  return q8_rows(ctx, w, x_dev, nullptr, 0.0f, y_dev, tokens);
 }
 
 int lgh_q8_norm_gemv_dev(lgh_ctx *ctx, const lgh_q8 *w, const float *norm_w_dev, float eps, const float *hidden_dev,
@@ -1103,16 +1146,7 @@ int lgh_q8_norm_gemv_dev(lgh_ctx *ctx, const lgh_q8 *w, const float *norm_w_dev,
   if (!aligned16(hidden_dev) || !aligned16(norm_w_dev))
     return fail(ctx, LGH_ERR_INVALID_ARG, "hidden and norm weight must be 16-byte aligned");
   if (int r = set_device(ctx)) return r;
-  const float *x = hidden_dev, *nw = w->k ? norm_w_dev : nullptr;
-  if (nw && w->k > lgh::kQ8GemvMaxK) {  // rows longer than the prologue covers: rms_norm first
-    if (int r = ensure(ctx, &ctx->ffn, &ctx->ffn_bytes, tokens * w->k * sizeof(float))) return r;
-    float *nd = static_cast<float *>(ctx->ffn);
-    LGH_HIP(ctx, lgh::launch_rms_norm(hidden_dev, nw, w->k, tokens, eps, nd, ctx->stream));
-    x = nd;
-    nw = nullptr;
-  }
-  LGH_HIP(ctx, lgh::launch_q8_gemv(w, x, y_dev, tokens, nw, eps, ctx->stream));
-  return LGH_OK;
+  return q8_rows(ctx, w, hidden_dev, w->k ? norm_w_dev : nullptr, eps, y_dev, tokens);
 }
 
 int lgh_q8_norm_gemv(lgh_ctx *ctx, const lgh_q8 *w, const float *norm_w, float eps, const float *hidden, float *y,

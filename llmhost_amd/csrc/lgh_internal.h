@@ -196,7 +196,10 @@ hipError_t launch_q4_gemv_batch(const lgh_q4 *w, const float *x, const int8_t *c
 //          K group g (0..3) holds codes 8g..8g+7 of the pair's two blocks
 //          (the B operand of v_mfma_i32_16x16x32_i8, 8 bytes per block);
 //   scales [mt][pq][16 tokens][4 blocks] f32.
-// Padding tokens and blocks hold 0.
+// Padding tokens and blocks hold 0.  That is MmaOrder::kBlock; kPair, for a
+// 64-deep MFMA over weights in natural order (the Q8_0 batch kernel), gives
+// lane (t, g) codes 16 (g % 2) .. + 15 of the pair's block g / 2.
+enum class MmaOrder : int { kBlock, kPair };
 struct Q4MmaPlan {
   int TT, KW, CB, RG;
   bool ok;
@@ -205,7 +208,8 @@ struct Q4MmaPlan {
 // route table prefers the GEMM (for matrices that cannot hold a GEMM image).
 Q4MmaPlan plan_q4_mma(size_t n, size_t m, size_t bpr, bool any_shape = false);
 hipError_t launch_act_quant_mma(const float *x, ActPrologue pro, size_t m, size_t k, int per_row, uint8_t *codes,
-                                float *scales, float *scratch, hipStream_t stream);
+                                float *scales, float *scratch, hipStream_t stream,
+                                MmaOrder order = MmaOrder::kBlock);
 // The same image from ActQ8 codes [m][k] and block scales [m][k/32].
 hipError_t launch_act_codes_mma(const int8_t *aq, const float *as, size_t m, size_t k, uint8_t *codes,
                                 float *scales, hipStream_t stream);
@@ -217,6 +221,13 @@ hipError_t launch_q4_gemv_mma(const lgh_q4 *w, const uint8_t *codes, const float
 constexpr size_t kQ8GemvMaxK = 32768;
 hipError_t launch_q8_gemv(const lgh_q8 *w, const float *x, float *y, size_t tokens, const float *norm_w, float eps,
                           hipStream_t stream);
+// The Q8_0 product of 1 <= m <= 64 tokens on the matrix cores (lgh_q8_batch.hip)
+// from the activation image of launch_act_quant_mma (kPair, per-block scales): one
+// pass over the weights.  q8_batch_wanted: whether a call of `tokens` tokens
+// takes it rather than the GEMV's pass per token.
+bool q8_batch_wanted(const lgh_q8 *w, size_t tokens);
+hipError_t launch_q8_mma(const lgh_q8 *w, const uint8_t *codes, const float *scales, float *y, size_t m,
+                         hipStream_t stream);
 
 // Batched activation quantization: x[m][k] -> qs[m][k], scales[m][k/32]
 // (+ sums if non-null).  row_scale: scratch of m floats (used for per_row).

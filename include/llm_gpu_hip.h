@@ -296,8 +296,9 @@ int lgh_silu_mul_dev(lgh_ctx *ctx, float *g_dev, const float *u_dev, size_t n);
  *   h      = silu(g) * u
  *   hidden = (float)((double)hidden + (double)(W2 h))   (gemv_q4_add / gemm_q4_add)
  * W1, W3: [inter, dim]; W2: [dim, inter].  Both activation quantizations
- * follow the context's act-quant mode.  One token with dim <= 2048 runs two
- * fused launches (the second reads h's ActQ8 codes written by the first).
+ * follow the context's act-quant mode.  1 to 4 tokens with dim <= 2048 run
+ * two fused launches (the second reads h's ActQ8 codes written by the first;
+ * PerRow, and a down projection outside their reach, pass h in f32).
  * Otherwise the ops above run on the device one after another, except that
  * for 5 or more tokens the norm and the gate/up activation image are
  * formed in one launch (the normed rows are not written) and the down
@@ -318,8 +319,8 @@ int lgh_q4_ffn_residual_dev(lgh_ctx *ctx, const lgh_q4 *w1, const lgh_q4 *w3, co
  * -- Lfm2::attn_decode's q_proj / k_proj / v_proj (crates/llm-engine/src/
  * lfm2.rs:784-794) and Lfm2::conv_update's in_proj (lfm2.rs:651-659); prefill
  * alike (lfm2.rs:698-711, and 609-625 when no position is padding).  Every W[j] has the same k; y[j] is
- * [tokens, W[j].n].  One token with k <= 2048 runs one launch: the norm in
- * its prologue and one activation quantization shared by all matrices (as
+ * [tokens, W[j].n].  1 to 4 tokens with k <= 2048 run one launch: the norm
+ * in its prologue and one activation quantization shared by all matrices (as
  * gemv_q4_pair shares one, crates/llm-cpu/src/gemv_q4.rs:396-443); otherwise
  * rms_norm then one lgh_q4_gemm per matrix (for 5 or more tokens the norm is
  * applied by the launch that writes the shared activation image).

@@ -895,11 +895,13 @@ static int materialize(lgh_ctx *ctx, const ActIn &in, size_t m, size_t k, const 
 
 // y[j] = x @ W[j]^T for 1..3 matrices with the same k, m rows of x: the
 // activation quantization of each route (the MMA image, the GEMM's operand
-// image) is done once and read by every matrix.  m == 1 and m <= 4 quantize
-// inside their kernels, per matrix.  The rows may be rms_norm(x) or
+// image) is done once and read by every matrix.  m == 1 quantizes inside its
+// kernel, per matrix; 2 <= m <= 4 once for all matrices, rows of up to 64 blocks
+// inside the kernel (with the norm).  The rows may be rms_norm(x) or
 // silu(x) * u (ActIn): the MMA and GEMM routes form them in the launch that
 // writes their activation image (the normed rows are never written), the
-// others after one more launch that writes them out.
+// others, where they do not norm in the kernel, after one more launch that
+// writes them out.
 static int gemm_multi_dev(lgh_ctx *ctx, const Ws &wsp, const lgh_q4 *const *w, int nmat, ActIn in,
                           float *const *y_dev, size_t m, int mode) {
   const size_t k = w[0]->k, bpr = w[0]->bpr;
@@ -924,6 +926,11 @@ static int gemm_multi_dev(lgh_ctx *ctx, const Ws &wsp, const lgh_q4 *const *w, i
   if (int r = set_device(ctx)) return r;
   // Small batches are weight-stream bound: nibble planes, no operand image.
   if (lgh::plan_q4_batch(m, bpr).ok) {  // m <= 4: dot4 on the nibble planes
+    if (!in.u && lgh::q4_batch_norms(bpr)) {  // the rows normed and quantized inside the kernel
+      LGH_HIP(ctx, lgh::launch_q4_gemv_batch(w, y_dev, nmat, in.x, nullptr, nullptr, in.nw, in.eps, m, mode,
+                                             ctx->act_mode, ctx->stream));
+      return LGH_OK;
+    }
     if (int r = materialize(ctx, in, m, k, &x_dev)) return r;
     if (lgh::q4_batch_quantize_once(bpr)) {  // long rows: x quantized once, shared by every matrix
       Carve cv;
@@ -934,13 +941,12 @@ static int gemm_multi_dev(lgh_ctx *ctx, const Ws &wsp, const lgh_q4 *const *w, i
       auto *sc = reinterpret_cast<float *>(ws + os);
       LGH_HIP(ctx, lgh::launch_act_quant(x_dev, m, k, ctx->act_mode, qs, sc, nullptr,
                                          reinterpret_cast<float *>(ws + orow), ctx->stream));
-      for (int j = 0; j < nmat; j++)
-        LGH_HIP(ctx, lgh::launch_q4_gemv_batch(w[j], nullptr, qs, sc, y_dev[j], m, mode, 0, ctx->stream));
+      LGH_HIP(ctx, lgh::launch_q4_gemv_batch(w, y_dev, nmat, nullptr, qs, sc, nullptr, 0.0f, m, mode, 0,
+                                             ctx->stream));
       return LGH_OK;
     }
-    for (int j = 0; j < nmat; j++)  // x quantized inside the kernel
-      LGH_HIP(ctx, lgh::launch_q4_gemv_batch(w[j], x_dev, nullptr, nullptr, y_dev[j], m, mode, ctx->act_mode,
-                                             ctx->stream));
+    LGH_HIP(ctx, lgh::launch_q4_gemv_batch(w, y_dev, nmat, x_dev, nullptr, nullptr, nullptr, 0.0f, m, mode,
+                                           ctx->act_mode, ctx->stream));
     return LGH_OK;
   }
   if (lgh::plan_q4_mma(nmax, m, bpr).ok) {  // m <= 64: activation image, then int8 MFMA per block
@@ -1292,25 +1298,33 @@ static int check_ffn(lgh_ctx *ctx, const lgh_q4 *w1, const lgh_q4 *w3, const lgh
   return LGH_OK;
 }
 
-// One token on a fused-shape FFN: two launches.
+// Up to kFfnMaxTokens tokens on a fused-shape FFN: two launches.
 static int ffn_fused(lgh_ctx *ctx, const lgh_q4 *w1, const lgh_q4 *w3, const lgh_q4 *w2, const float *norm_w_dev,
-                     float eps, float *hidden_dev) {
+                     float eps, float *hidden_dev, size_t m) {
   const size_t n = w1->n;
-  // PerBlock and a GEMV-sized W2: h leaves the gate/up kernel already
-  // quantized.  Otherwise (PerRow needs all of h for its scale, or K beyond
-  // the GEMV) h goes out in f32 through the regular M = 1 path.
-  const bool codes = ctx->act_mode == LGH_ACT_PER_BLOCK && lgh::plan_q4_gemv(w2->n, w2->bpr, 1).ok;
+  // PerBlock and a W2 whose kernel takes codes: h leaves the gate/up kernel
+  // already quantized.  Otherwise (PerRow needs all of h for its scale, or
+  // rows the kernels do not take) h goes out in f32 through the regular path.
+  const bool codes = ctx->act_mode == LGH_ACT_PER_BLOCK &&
+                     (m == 1 ? lgh::plan_q4_gemv(w2->n, w2->bpr, 1).ok
+                             : lgh::plan_q4_batch(m, w2->bpr).ok && lgh::q4_batch_quantize_once(w2->bpr));
   Carve cv;
-  const size_t o_q = cv.take(n), o_s = cv.take(n / 32 * sizeof(float)), o_f = cv.take(codes ? 0 : n * sizeof(float));
+  const size_t o_q = cv.take(m * n), o_s = cv.take(m * (n / 32) * sizeof(float));
+  const size_t o_f = cv.take(codes ? 0 : m * n * sizeof(float));
   if (int r = ensure(ctx, &ctx->ffn, &ctx->ffn_bytes, cv.off)) return r;
   char *f = static_cast<char *>(ctx->ffn);
   auto *hq = reinterpret_cast<int8_t *>(f + o_q);
   auto *hs = reinterpret_cast<float *>(f + o_s);
   auto *hf = reinterpret_cast<float *>(f + o_f);
-  LGH_HIP(ctx, lgh::launch_ffn_gate_up(w1, w3, hidden_dev, norm_w_dev, eps, ctx->act_mode, codes ? hq : nullptr, hs,
-                                       codes ? nullptr : hf, nullptr, nullptr, ctx->stream));
-  if (!codes) return lgh_q4_gemm_dev(ctx, w2, hf, hidden_dev, 1, LGH_ADD_F64);
-  LGH_HIP(ctx, lgh::launch_q4_gemv_codes(w2, hq, hs, hidden_dev, LGH_ADD_F64, ctx->stream));
+  LGH_HIP(ctx, lgh::launch_ffn_gate_up(w1, w3, hidden_dev, norm_w_dev, eps, m, ctx->act_mode, codes ? hq : nullptr,
+                                       hs, codes ? nullptr : hf, nullptr, nullptr, ctx->stream));
+  if (!codes) return lgh_q4_gemm_dev(ctx, w2, hf, hidden_dev, m, LGH_ADD_F64);
+  if (m == 1) {
+    LGH_HIP(ctx, lgh::launch_q4_gemv_codes(w2, hq, hs, hidden_dev, LGH_ADD_F64, ctx->stream));
+  } else {
+    LGH_HIP(ctx, lgh::launch_q4_gemv_batch(&w2, &hidden_dev, 1, nullptr, hq, hs, nullptr, 0.0f, m, LGH_ADD_F64, 0,
+                                           ctx->stream));
+  }
   return LGH_OK;
 }
 
@@ -1324,7 +1338,8 @@ int lgh_q4_ffn_residual_dev(lgh_ctx *ctx, const lgh_q4 *w1, const lgh_q4 *w3, co
   if (!aligned16(hidden_dev) || !aligned16(norm_w_dev))
     return fail(ctx, LGH_ERR_INVALID_ARG, "hidden and norm weight must be 16-byte aligned");
   if (int r = set_device(ctx)) return r;
-  if (tokens == 1 && lgh::ffn_gate_up_supported(w1)) return ffn_fused(ctx, w1, w3, w2, norm_w_dev, eps, hidden_dev);
+  if (tokens <= lgh::kFfnMaxTokens && lgh::ffn_gate_up_supported(w1))
+    return ffn_fused(ctx, w1, w3, w2, norm_w_dev, eps, hidden_dev, tokens);
   // Several tokens (or a wide model): the reference's sequence of ops
   // (lfm2.rs:861-881) on the device, intermediates in the context.  The norm
   // and silu(g) * u are formed inside the activation-image kernels of the
@@ -1387,7 +1402,7 @@ int lgh_q4_ffn_gate_up(lgh_ctx *ctx, const lgh_q4 *w1, const lgh_q4 *w3, const f
   auto *qd = reinterpret_cast<int8_t *>(st + oq);
   LGH_HIP(ctx, hipMemcpyAsync(xd, hidden, xb, hipMemcpyHostToDevice, ctx->stream));
   if (norm_w) LGH_HIP(ctx, hipMemcpyAsync(nd, norm_w, xb, hipMemcpyHostToDevice, ctx->stream));
-  LGH_HIP(ctx, lgh::launch_ffn_gate_up(w1, w3, xd, nd, eps, ctx->act_mode, qd, sd, hd, gd, ud, ctx->stream));
+  LGH_HIP(ctx, lgh::launch_ffn_gate_up(w1, w3, xd, nd, eps, 1, ctx->act_mode, qd, sd, hd, gd, ud, ctx->stream));
   LGH_HIP(ctx, hipMemcpyAsync(g, gd, yb, hipMemcpyDeviceToHost, ctx->stream));
   LGH_HIP(ctx, hipMemcpyAsync(u, ud, yb, hipMemcpyDeviceToHost, ctx->stream));
   LGH_HIP(ctx, hipMemcpyAsync(h, hd, yb, hipMemcpyDeviceToHost, ctx->stream));

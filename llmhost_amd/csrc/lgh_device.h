@@ -382,10 +382,45 @@ __device__ __forceinline__ void rms_norm_regs(float4 (&xv)[XJ], const float4 (&n
   }
 }
 
+// rms_norm_regs for T token rows held in registers, one barrier for them all.
+template <int THREADS, int T, int XJ>
+__device__ __forceinline__ void rms_norm_tokens(float4 (&xv)[T][XJ], const float4 (&nv)[XJ], double inv_k, float eps,
+                                                double (&s_ss)[T][THREADS / kWave]) {
+#pragma unroll
+  for (int t = 0; t < T; t++) {
+    double ss = 0.0;
+#pragma unroll
+    for (int j = 0; j < XJ; j++) {
+      const double x0 = xv[t][j].x, x1 = xv[t][j].y, x2 = xv[t][j].z, x3 = xv[t][j].w;
+      ss += x0 * x0;
+      ss += x1 * x1;
+      ss += x2 * x2;
+      ss += x3 * x3;
+    }
+    ss = wave_sum_dpp64(ss);
+    if ((threadIdx.x & (kWave - 1)) == 0) s_ss[t][threadIdx.x / kWave] = ss;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < T; t++) {
+    double tot = 0.0;
+#pragma unroll
+    for (int i = 0; i < THREADS / kWave; i++) tot += s_ss[t][i];
+    const float scale = rms_scale(tot, inv_k, eps);
+#pragma unroll
+    for (int j = 0; j < XJ; j++) {
+      xv[t][j].x = nv[j].x * (xv[t][j].x * scale);
+      xv[t][j].y = nv[j].y * (xv[t][j].y * scale);
+      xv[t][j].z = nv[j].z * (xv[t][j].z * scale);
+      xv[t][j].w = nv[j].w * (xv[t][j].w * scale);
+    }
+  }
+}
+
 // ---- x -> LDS codes, shared by the GEMV-style kernels --------------------
 // Quantize the float4s held in registers (thread t holds x4[t + THREADS j])
-// into LDS: s_qs (natural order) and s_sa, for blocks [0, nblk).  All
-// threads must call it; it ends with a barrier.
+// into LDS: s_qs (natural order) and s_sa, for blocks [0, nblk).  The caller
+// puts a barrier behind it.
 template <int THREADS, int XJ>
 __device__ __forceinline__ void quant_regs(const float4 (&xv)[XJ], int nblk, bool per_row, float row_scale,
                                            int8_t *s_qs, float *s_sa) {
@@ -402,7 +437,6 @@ __device__ __forceinline__ void quant_regs(const float4 (&xv)[XJ], int nblk, boo
       if (g == 0) s_sa[b] = scale;
     }
   }
-  __syncthreads();
 }
 
 // Row amax / 127 over the register-resident x (PerRow), or 0.
@@ -426,6 +460,21 @@ __device__ __forceinline__ void quantize_regs_to_lds(const float4 (&xv)[XJ], int
                                                      float *s_sa, float *s_red) {
   const float rs = row_scale_of<THREADS, XJ>(xv, per_row, s_red);
   quant_regs<THREADS, XJ>(xv, bpr, per_row != 0, rs, s_qs, s_sa);
+  __syncthreads();
+}
+
+// The same for T token rows (PerRow: one barrier per row for its amax; s_red
+// [T][waves]), one barrier behind them all.
+template <int THREADS, int T, int XJ>
+__device__ __forceinline__ void quantize_tokens_to_lds(const float4 (&xv)[T][XJ], int bpr, int per_row, int8_t *s_qs,
+                                                       int qs_stride, float *s_sa, int sa_stride,
+                                                       float (&s_red)[T][THREADS / kWave]) {
+#pragma unroll
+  for (int t = 0; t < T; t++) {
+    const float rs = row_scale_of<THREADS, XJ>(xv[t], per_row, s_red[t]);
+    quant_regs<THREADS, XJ>(xv[t], bpr, per_row != 0, rs, s_qs + t * qs_stride, s_sa + t * sa_stride);
+  }
+  __syncthreads();
 }
 
 // x -> LDS codes with 4-lane groups: thread t holds the 32-byte chunks

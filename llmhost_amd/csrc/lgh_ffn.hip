@@ -1,4 +1,4 @@
-// Decode-step SwiGLU FFN residual block for gfx950, one token (replaces
+// Decode-step SwiGLU FFN residual block for gfx950, up to 4 tokens (replaces
 // Lfm2::ffn_residual_in, crates/llm-engine/src/lfm2.rs:883-911):
 //   normed = rms_norm(hidden, ffn_norm)          crates/llm-cpu/src/ops.rs:8-23
 //   g, u   = W1 normed, W3 normed                gemv_q4_pair, gemv_q4.rs:396-443
@@ -10,8 +10,8 @@
 //     W1 and the same 32 rows of W3 (one row of each per 16-lane DPP row),
 //     then silu(g) * u for those 32 rows -- exactly one 32-element block of
 //     h -- and that block's ActQ8 codes and scale;
-//   * the down GEMV reading those codes (q4_gemv_kernel, PREQ), AddF64 into
-//     hidden.
+//   * the down GEMV reading those codes (q4_gemv_kernel or, for 2 to 4 tokens,
+//     q4_gemv_batch_kernel, PREQ), AddF64 into hidden.
 // The down GEMV therefore skips loading 4*inter bytes of h and quantizing it
 // in every workgroup, which is the prologue that bounds the plain GEMV at
 // K = 8192.
@@ -39,23 +39,32 @@ struct FfnUpArgs {
   double inv_k;     // 1 / k in f64 (ops.rs:12)
   float eps;
   int bpr;        // k / 32
+  int n;          // rows of W1 and W3
+  int m;          // tokens: x is [m][k], the outputs [m][n]
   int per_row;    // ActQ8 mode for `normed`
-  int8_t *hq;     // ActQ8 (PerBlock) codes of h [n], or null
-  float *hs;      // their scales [n / 32]
-  float *hf;      // h [n], or null
-  float *g_out;   // g [n], or null
-  float *u_out;   // u [n], or null
+  int8_t *hq;     // ActQ8 (PerBlock) codes of h, or null
+  float *hs;      // their scales [m][n / 32]
+  float *hf;      // h, or null
+  float *g_out;   // g, or null
+  float *u_out;   // u, or null
 };
 
-template <int BPL>
+// T token slots (those past m read zeros and store nothing): each weight block
+// is unpacked once and dotted with the T rows' codes, as q4_gemv_batch_kernel
+// does, in the same order.  Bound by the launch, one round trip and the weight
+// stream, so launches count: the block of 2 / 3 / 4 tokens, against the sequence
+// (rms_norm, gate, up, silu, act_quant, down): dim 2048, inter 8192 27.4 / 28.0 /
+// 28.5 -> 14.8 / 17.0 / 17.1 us; dim 1024, inter 4608 21.0 / 21.3 / 21.8 -> 11.1 /
+// 12.9 / 13.0 us; bit-identical.
+template <int T, int BPL>
 __global__ __launch_bounds__(kFfnThreads) void ffn_gate_up_kernel(FfnUpArgs a) {
   constexpr int KB = 16 * BPL;  // blocks covered (>= bpr)
   constexpr int XJ = (KB * 8 + kFfnThreads - 1) / kFfnThreads;
-  __shared__ __align__(16) int8_t s_qs[KB * 32];
-  __shared__ float s_sa[KB];
-  __shared__ float s_red[kFfnWaves];
-  __shared__ double s_ss[kFfnWaves];
-  __shared__ __align__(16) float s_h[32];
+  __shared__ __align__(16) int8_t s_qs[T][KB * 32];
+  __shared__ float s_sa[T][KB];
+  __shared__ float s_red[T][kFfnWaves];
+  __shared__ double s_ss[T][kFfnWaves];
+  __shared__ __align__(16) float s_h[T][32];
   const int bpr = a.bpr;
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
@@ -65,14 +74,17 @@ __global__ __launch_bounds__(kFfnThreads) void ffn_gate_up_kernel(FfnUpArgs a) {
   const int r = lane >> 4, c = lane & 15;
 
   // (1) hidden and the norm weight (elements >= k read as 0).
-  const auto xr = make_rsrc(a.x, static_cast<uint32_t>(bpr) * 128u);
   const auto nr = make_rsrc(a.nw, a.nw ? static_cast<uint32_t>(bpr) * 128u : 0u);
-  float4 xv[XJ], nv[XJ];
+  float4 xv[T][XJ], nv[XJ];
 #pragma unroll
-  for (int j = 0; j < XJ; j++) {
-    xv[j] = buf_load_f4(xr, static_cast<uint32_t>(tid + j * kFfnThreads) * 16u);
-    nv[j] = buf_load_f4(nr, static_cast<uint32_t>(tid + j * kFfnThreads) * 16u);
+  for (int t = 0; t < T; t++) {
+    const auto xr =
+        make_rsrc(a.x + static_cast<size_t>(t) * bpr * 32, t < a.m ? static_cast<uint32_t>(bpr) * 128u : 0u);
+#pragma unroll
+    for (int j = 0; j < XJ; j++) xv[t][j] = buf_load_f4(xr, static_cast<uint32_t>(tid + j * kFfnThreads) * 16u);
   }
+#pragma unroll
+  for (int j = 0; j < XJ; j++) nv[j] = buf_load_f4(nr, static_cast<uint32_t>(tid + j * kFfnThreads) * 16u);
   // (1b) The norm and the quantization wait for every wave's hidden: queue
   // those requests before any wave's weight requests.
   __builtin_amdgcn_sched_barrier(0);
@@ -100,76 +112,74 @@ __global__ __launch_bounds__(kFfnThreads) void ffn_gate_up_kernel(FfnUpArgs a) {
   // (3) RMSNorm (ops.rs:8-23): sum of squares in f64, scale =
   // f32(1 / sqrt(sumsq * (1/dim) + eps)) in f64, normed = w * (x * scale) in
   // f32.  The f64 sum is a fixed tree instead of the reference's sequence.
-  if (a.nw) {
-    double ss = 0.0;
-#pragma unroll
-    for (int j = 0; j < XJ; j++) {
-      const double x0 = xv[j].x, x1 = xv[j].y, x2 = xv[j].z, x3 = xv[j].w;
-      ss += x0 * x0;
-      ss += x1 * x1;
-      ss += x2 * x2;
-      ss += x3 * x3;
-    }
-    ss = wave_sum_dpp64(ss);
-    if (lane == 0) s_ss[wave] = ss;
-    __syncthreads();
-    double tot = 0.0;
-#pragma unroll
-    for (int i = 0; i < kFfnWaves; i++) tot += s_ss[i];
-    const float scale = rms_scale(tot, a.inv_k, a.eps);
-#pragma unroll
-    for (int j = 0; j < XJ; j++) {
-      xv[j].x = nv[j].x * (xv[j].x * scale);
-      xv[j].y = nv[j].y * (xv[j].y * scale);
-      xv[j].z = nv[j].z * (xv[j].z * scale);
-      xv[j].w = nv[j].w * (xv[j].w * scale);
-    }
-  }
+  if (a.nw) rms_norm_tokens<kFfnThreads, T, XJ>(xv, nv, a.inv_k, a.eps, s_ss);
 
   // (4) ActQ8 of normed into LDS, shared by both matrices.
-  quantize_regs_to_lds<kFfnThreads, XJ>(xv, bpr, a.per_row, s_qs, s_sa, s_red);
+  quantize_tokens_to_lds<kFfnThreads, T, XJ>(xv, bpr, a.per_row, &s_qs[0][0], KB * 32, &s_sa[0][0], KB, s_red);
 
   // (5) dots + fold for both rows (branch-free: blocks past the row add
   // exactly 0), DPP row sums, then g, u and h of the lane's row.
-  float ag = 0.0f, au = 0.0f;
+  float ag[T], au[T];
+#pragma unroll
+  for (int t = 0; t < T; t++) ag[t] = au[t] = 0.0f;
 #pragma unroll
   for (int j = 0; j < BPL; j++) {
     const int kb = c + 16 * j;
     const int kbc = kb < bpr ? kb : 0;
-    const v4i *ap = reinterpret_cast<const v4i *>(s_qs + kbc * 32);
-    const v4i a0 = ap[0], a1 = ap[1];
-    const float sa = s_sa[kbc];
-    ag = fmaf(static_cast<float>(dot_q4_block16(w1[j], a0, a1)), h2f(s1[j]) * sa, ag);
-    au = fmaf(static_cast<float>(dot_q4_block16(w3[j], a0, a1)), h2f(s3[j]) * sa, au);
+    const float sw1 = h2f(s1[j]), sw3 = h2f(s3[j]);
+#pragma unroll
+    for (int t = 0; t < T; t++) {
+      const v4i *ap = reinterpret_cast<const v4i *>(&s_qs[t][kbc * 32]);
+      const v4i a0 = ap[0], a1 = ap[1];
+      const float sa = s_sa[t][kbc];
+      ag[t] = fmaf(static_cast<float>(dot_q4_block16(w1[j], a0, a1)), sw1 * sa, ag[t]);
+      au[t] = fmaf(static_cast<float>(dot_q4_block16(w3[j], a0, a1)), sw3 * sa, au[t]);
+    }
   }
-  ag += dpp<0xB1>(ag);
-  au += dpp<0xB1>(au);
-  ag += dpp<0x4E>(ag);
-  au += dpp<0x4E>(au);
-  ag += dpp<0x141>(ag);
-  au += dpp<0x141>(au);
-  ag += dpp<0x140>(ag);
-  au += dpp<0x140>(au);
-  if (c == 0) {
+#pragma unroll
+  for (int t = 0; t < T; t++) {
+    ag[t] += dpp<0xB1>(ag[t]);
+    au[t] += dpp<0xB1>(au[t]);
+    ag[t] += dpp<0x4E>(ag[t]);
+    au[t] += dpp<0x4E>(au[t]);
+    ag[t] += dpp<0x141>(ag[t]);
+    au[t] += dpp<0x141>(au[t]);
+    ag[t] += dpp<0x140>(ag[t]);
+    au[t] += dpp<0x140>(au[t]);
+  }
+  // Every lane of a DPP row holds the row's sums: lane c takes token c.
+  float gs = ag[0], us = au[0];
+#pragma unroll
+  for (int t = 1; t < T; t++) {
+    gs = c == t ? ag[t] : gs;
+    us = c == t ? au[t] : us;
+  }
+  if (c < T) {
     const int i = wave * 4 + r;
-    const float g = ag * 0.0625f, u = au * 0.0625f;  // exact: undo the x16 of the unpack
+    const float g = gs * 0.0625f, u = us * 0.0625f;  // exact: undo the x16 of the unpack
     const float h = silu_mul1(g, u);
-    s_h[i] = h;
-    if (a.g_out) a.g_out[base + i] = g;
-    if (a.u_out) a.u_out[base + i] = u;
-    if (a.hf) a.hf[base + i] = h;
+    s_h[c][i] = h;
+    if (c < a.m) {
+      const size_t o = static_cast<size_t>(c) * a.n + base + i;
+      if (a.g_out) a.g_out[o] = g;
+      if (a.u_out) a.u_out[o] = u;
+      if (a.hf) a.hf[o] = h;
+    }
   }
-  // (6) the block of h: its ActQ8 codes and scale (8 lanes, as
+  // (6) each token's block of h: its ActQ8 codes and scale (8 lanes, as
   // act_quant_kernel).
   if (!a.hq) return;  // uniform
   __syncthreads();
-  if (wave == 0 && lane < 8) {
-    const float4 hv = reinterpret_cast<const float4 *>(s_h)[lane];
+  const int t = lane >> 3;
+  if (wave == 0 && t < T) {
+    const float4 hv = reinterpret_cast<const float4 *>(s_h[t])[lane & 7];
     float scale;
     int sum;
     const int q = act_quant_group8(hv, false, 0.0f, scale, sum);
-    reinterpret_cast<int *>(a.hq + base)[lane] = q;
-    if (lane == 0) a.hs[blockIdx.x] = scale;
+    if (t < a.m) {
+      reinterpret_cast<int *>(a.hq + static_cast<size_t>(t) * a.n + base)[lane & 7] = q;
+      if ((lane & 7) == 0) a.hs[static_cast<size_t>(t) * (a.n / 32) + blockIdx.x] = scale;
+    }
   }
 }
 
@@ -207,10 +217,20 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(float *__restrict__ g, co
   g[i] = silu_mul1(g[i], u[i]);
 }
 
-template <int BPL>
+template <int T, int BPL>
 hipError_t launch_gate_up(const FfnUpArgs &a, int wgs, hipStream_t st) {
-  hipLaunchKernelGGL(ffn_gate_up_kernel<BPL>, dim3(wgs), dim3(kFfnThreads), 0, st, a);
+  hipLaunchKernelGGL((ffn_gate_up_kernel<T, BPL>), dim3(wgs), dim3(kFfnThreads), 0, st, a);
   return hipGetLastError();
+}
+
+template <int T>
+hipError_t dispatch_gate_up(const FfnUpArgs &a, int wgs, hipStream_t st) {
+  switch ((a.bpr + 15) / 16) {
+    case 1: return launch_gate_up<T, 1>(a, wgs, st);
+    case 2: return launch_gate_up<T, 2>(a, wgs, st);
+    case 3: return launch_gate_up<T, 3>(a, wgs, st);
+    default: return launch_gate_up<T, 4>(a, wgs, st);
+  }
 }
 
 }  // namespace
@@ -218,19 +238,16 @@ hipError_t launch_gate_up(const FfnUpArgs &a, int wgs, hipStream_t st) {
 bool ffn_gate_up_supported(const lgh_q4 *w1) { return w1->bpr >= 1 && w1->bpr <= kFfnMaxBpr && w1->n % 32 == 0; }
 
 hipError_t launch_ffn_gate_up(const lgh_q4 *w1, const lgh_q4 *w3, const float *x, const float *norm_w, float eps,
-                              int per_row, int8_t *hq, float *hs, float *hf, float *g, float *u,
+                              size_t m, int per_row, int8_t *hq, float *hs, float *hf, float *g, float *u,
                               hipStream_t st) {
-  if (!ffn_gate_up_supported(w1)) return hipErrorInvalidValue;
+  if (!ffn_gate_up_supported(w1) || m < 1 || m > kFfnMaxTokens) return hipErrorInvalidValue;
   if (w1->n == 0) return hipSuccess;
   const FfnUpArgs a{w1->qs, w3->qs, w1->sc, w3->sc, x, norm_w, 1.0 / static_cast<double>(w1->k), eps,
-                    static_cast<int>(w1->bpr), per_row, hq, hs, hf, g, u};
+                    static_cast<int>(w1->bpr), static_cast<int>(w1->n), static_cast<int>(m), per_row, hq, hs, hf, g,
+                    u};
   const int wgs = static_cast<int>(w1->n / 32);
-  switch ((w1->bpr + 15) / 16) {
-    case 1: return launch_gate_up<1>(a, wgs, st);
-    case 2: return launch_gate_up<2>(a, wgs, st);
-    case 3: return launch_gate_up<3>(a, wgs, st);
-    default: return launch_gate_up<4>(a, wgs, st);
-  }
+  if (m == 1) return dispatch_gate_up<1>(a, wgs, st);
+  return m == 2 ? dispatch_gate_up<2>(a, wgs, st) : dispatch_gate_up<4>(a, wgs, st);
 }
 
 hipError_t launch_rms_norm(const float *x, const float *w, size_t dim, size_t rows, float eps, float *out,

@@ -279,19 +279,28 @@ hipError_t dispatch_q4(const Q4GemvArgs &a, int total_wgs, bool preq, bool norm,
 // tokens), then reads each 18-byte nibble block once and dots it against the
 // T code rows in LDS: one nibble unpack, then 8 v_dot4_i32_i8 and one fold per
 // token.  Row mapping, slices and DPP row sums as in q4_gemv_kernel.
+// Up to three matrices with the same k share the launch and its quantization
+// (norm + q / k / v of 4 tokens, K=2048, 2048 + 2 x 512 rows: four launches 17.9
+// us, one 6.5 us): workgroups [0, wgs0) cover matrix 0, the next wgs1 matrix 1, the rest matrix 2.
 struct Q4BatchArgs {
-  const uint8_t *qs;
-  const uint16_t *sc;
+  const uint8_t *qs[3];
+  const uint16_t *sc[3];
+  float *y[3];  // [m][n[j]]
+  int n[3];
+  int wgs0, wgs1;
   const float *x;    // f32 [m][k]
   const int8_t *aq;  // PREQ: ActQ8 codes [m][k] and scales [m][k/32] instead of x
   const float *as;
-  float *y;  // [m][n]
-  int n, bpr, m, mode, per_row;
+  const float *nw;   // NORM: rms_norm weight [k]
+  double inv_k;      // NORM: 1 / k in f64 (ops.rs:12)
+  float eps;
+  int bpr, m, mode, per_row;
 };
 
 // PREQ: the T rows arrive already quantized (act_quant_kernel, once for
-// every workgroup) instead of each workgroup quantizing all of them.
-template <int T, int BPL, int KW, int W, bool PREQ>
+// every workgroup) instead of each workgroup quantizing all of them.  NORM:
+// the rows are rms_norm'd first, as in q4_gemv_kernel.
+template <int T, int BPL, int KW, int W, bool PREQ, bool NORM>
 __global__ __launch_bounds__(W * kWave) void q4_gemv_batch_kernel(Q4BatchArgs a) {
   constexpr int THREADS = W * kWave;
   constexpr int KB = 16 * BPL * KW;
@@ -300,17 +309,30 @@ __global__ __launch_bounds__(W * kWave) void q4_gemv_batch_kernel(Q4BatchArgs a)
   constexpr int QJ = PREQ ? (KB * 2 + THREADS - 1) / THREADS : 1;  // 16-byte code chunks per thread and row
   constexpr int SJ = PREQ ? (KB + THREADS - 1) / THREADS : 1;      // block scales per thread and row
   static_assert(W % KW == 0, "slices divide the waves");
+  static_assert(!(PREQ && NORM), "the norm needs x");
   __shared__ __align__(16) int8_t s_qs[T][KB * 32];
   __shared__ float s_sa[T][KB];
-  __shared__ float s_red[W];
+  __shared__ float s_red[T][W];
+  __shared__ double s_ss[T][NORM ? W : 1];
   __shared__ float s_part[KW > 1 ? RG * 4 * KW * T : 1];
   const int bpr = a.bpr;
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = uniform(tid / kWave);
   const int rg = wave / KW, ks = wave % KW;
-  const int row0 = (blockIdx.x * RG + rg) * 4;
-  const int rows = uniform(max(0, min(4, a.n - row0)));
+  int wg = blockIdx.x, mat = 0;
+  if (wg >= a.wgs0) {
+    wg -= a.wgs0;
+    mat = 1;
+    if (wg >= a.wgs1) {
+      wg -= a.wgs1;
+      mat = 2;
+    }
+  }
+  const int n = a.n[mat];
+  float *const y = a.y[mat];
+  const int row0 = (wg * RG + rg) * 4;
+  const int rows = uniform(max(0, min(4, n - row0)));
   const int r = lane >> 4, c = lane & 15;
   const int kb0 = ks * 16 * BPL + c;
 
@@ -318,6 +340,12 @@ __global__ __launch_bounds__(W * kWave) void q4_gemv_batch_kernel(Q4BatchArgs a)
   // read as 0), issued before the weights so that waiting for them leaves the
   // weight loads in flight.
   float4 xv[T][XJ];
+  float4 nv[NORM ? XJ : 1];
+  if constexpr (NORM) {
+    const auto nr = make_rsrc(a.nw, static_cast<uint32_t>(bpr) * 128u);
+#pragma unroll
+    for (int j = 0; j < XJ; j++) nv[j] = buf_load_f4(nr, static_cast<uint32_t>(tid + j * THREADS) * 16u);
+  }
   uint4 qv[T][QJ];
   float sv[T][SJ];
 #pragma unroll
@@ -340,8 +368,8 @@ __global__ __launch_bounds__(W * kWave) void q4_gemv_batch_kernel(Q4BatchArgs a)
   // (1b) PREQ over four or more K slices: every wave's code requests before
   // any wave's weight requests (M=2 / 4, K=8192, N=2048: 7.41 / 7.49 ->
   // 7.26 / 7.32 us; the x path at K=2048 and the codes at K=4096 measured
-  // no gain or a loss, interleaved A/B).
-  if constexpr (PREQ && KW >= 4) {
+  // no gain or a loss, interleaved A/B).  NORM waits for all of x, as the GEMV's.
+  if constexpr ((PREQ && KW >= 4) || NORM) {
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
@@ -349,8 +377,8 @@ __global__ __launch_bounds__(W * kWave) void q4_gemv_batch_kernel(Q4BatchArgs a)
 
   // (2) every weight load of this lane (rows past n read as 0).
   const size_t blk0 = static_cast<size_t>(row0) * bpr;
-  const auto wr = make_rsrc(a.qs + blk0 * 16, static_cast<uint32_t>(rows * bpr) * 16u);
-  const auto swr = make_rsrc(a.sc + blk0, static_cast<uint32_t>(rows * bpr) * 2u);
+  const auto wr = make_rsrc(a.qs[mat] + blk0 * 16, static_cast<uint32_t>(rows * bpr) * 16u);
+  const auto swr = make_rsrc(a.sc[mat] + blk0, static_cast<uint32_t>(rows * bpr) * 2u);
   uint4 w[BPL];
   uint16_t s[BPL];
 #pragma unroll
@@ -378,11 +406,8 @@ __global__ __launch_bounds__(W * kWave) void q4_gemv_batch_kernel(Q4BatchArgs a)
     }
     __syncthreads();
   } else {
-#pragma unroll
-    for (int t = 0; t < T; t++) {
-      const float rs = row_scale_of<THREADS, XJ>(xv[t], a.per_row, s_red);
-      quant_regs<THREADS, XJ>(xv[t], bpr, a.per_row != 0, rs, s_qs[t], s_sa[t]);
-    }
+    if constexpr (NORM) rms_norm_tokens<THREADS, T, XJ>(xv, nv, a.inv_k, a.eps, s_ss);
+    quantize_tokens_to_lds<THREADS, T, XJ>(xv, bpr, a.per_row, &s_qs[0][0], KB * 32, &s_sa[0][0], KB, s_red);
   }
 
   // (4) per block: one unpack, then T dots and folds.
@@ -423,7 +448,7 @@ __global__ __launch_bounds__(W * kWave) void q4_gemv_batch_kernel(Q4BatchArgs a)
     if (c == 0 && r < rows) {
 #pragma unroll
       for (int t = 0; t < T; t++)
-        if (t < a.m) store_row(a.y + static_cast<size_t>(t) * a.n, row0 + r, acc[t], a.mode);
+        if (t < a.m) store_row(y + static_cast<size_t>(t) * n, row0 + r, acc[t], a.mode);
     }
   } else {
     if (c == 0) {
@@ -437,18 +462,27 @@ __global__ __launch_bounds__(W * kWave) void q4_gemv_batch_kernel(Q4BatchArgs a)
         float sum = 0.0f;
 #pragma unroll
         for (int k = 0; k < KW; k++) sum += s_part[((rg * 4 + rr) * T + t) * KW + k];
-        store_row(a.y + static_cast<size_t>(t) * a.n, row0 + rr, sum, a.mode);
+        store_row(y + static_cast<size_t>(t) * n, row0 + rr, sum, a.mode);
       }
     }
   }
 }
 
 template <int BPL, int KW, bool PREQ = false>
-hipError_t launch_batch(const Q4BatchArgs &a, hipStream_t st) {
-  constexpr int W = 8;
-  const int rows_per_wg = 4 * W / KW;
-  const unsigned wgs = static_cast<unsigned>((a.n + rows_per_wg - 1) / rows_per_wg);
-  hipLaunchKernelGGL((q4_gemv_batch_kernel<4, BPL, KW, W, PREQ>), dim3(wgs), dim3(W * kWave), 0, st, a);
+hipError_t launch_batch(Q4BatchArgs a, hipStream_t st) {
+  constexpr int W = 8, kRows = 4 * W / KW;
+  const int wgs[3] = {(a.n[0] + kRows - 1) / kRows, (a.n[1] + kRows - 1) / kRows, (a.n[2] + kRows - 1) / kRows};
+  a.wgs0 = wgs[0];
+  a.wgs1 = wgs[1];
+  const dim3 grid(static_cast<unsigned>(wgs[0] + wgs[1] + wgs[2])), blk(W * kWave);
+  if constexpr (KW == 1 && !PREQ) {
+    if (a.nw) {
+      hipLaunchKernelGGL((q4_gemv_batch_kernel<4, BPL, KW, W, false, true>), grid, blk, 0, st, a);
+      return hipGetLastError();
+    }
+  }
+  if (a.nw) return hipErrorInvalidValue;  // q4_batch_norms
+  hipLaunchKernelGGL((q4_gemv_batch_kernel<4, BPL, KW, W, PREQ, false>), grid, blk, 0, st, a);
   return hipGetLastError();
 }
 
@@ -1099,13 +1133,32 @@ Q4BatchPlan plan_q4_batch(size_t m, size_t bpr) {
 // 8.25 / 8.90 -> 8.04 / 8.37 us.
 bool q4_batch_quantize_once(size_t bpr) { return bpr > 64; }
 
-hipError_t launch_q4_gemv_batch(const lgh_q4 *w, const float *x, const int8_t *codes, const float *scales, float *y,
-                                size_t m, int mode, int per_row, hipStream_t st) {
-  const Q4BatchPlan p = plan_q4_batch(m, w->bpr);
+bool q4_batch_norms(size_t bpr) { return bpr <= 64; }
+
+hipError_t launch_q4_gemv_batch(const lgh_q4 *const *w, float *const *y, int nmat, const float *x,
+                                const int8_t *codes, const float *scales, const float *norm_w, float eps, size_t m,
+                                int mode, int per_row, hipStream_t st) {
+  if (nmat < 1 || nmat > 3) return hipErrorInvalidValue;
+  const Q4BatchPlan p = plan_q4_batch(m, w[0]->bpr);
   if (!p.ok) return hipErrorInvalidValue;
-  if (w->n == 0) return hipSuccess;
-  Q4BatchArgs a{w->qs,  w->sc, x, codes, scales, y, static_cast<int>(w->n), static_cast<int>(w->bpr),
-                static_cast<int>(m), mode, per_row};
+  if (gemv_multi_rows(w, nmat) == 0) return hipSuccess;
+  Q4BatchArgs a{};
+  for (int j = 0; j < nmat; j++) {
+    a.qs[j] = w[j]->qs;
+    a.sc[j] = w[j]->sc;
+    a.y[j] = y[j];
+    a.n[j] = static_cast<int>(w[j]->n);
+  }
+  a.x = x;
+  a.aq = codes;
+  a.as = scales;
+  a.nw = norm_w;
+  a.inv_k = 1.0 / static_cast<double>(w[0]->k);
+  a.eps = eps;
+  a.bpr = static_cast<int>(w[0]->bpr);
+  a.m = static_cast<int>(m);
+  a.mode = mode;
+  a.per_row = per_row;
   if (codes) {
     if (p.KW == 1) return hipErrorInvalidValue;
     return p.KW == 2 ? launch_batch<4, 2, true>(a, st) : launch_batch<4, 4, true>(a, st);

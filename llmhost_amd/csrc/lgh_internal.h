@@ -145,16 +145,17 @@ int gemv_plans_uncovered();
 bool q4_gemv_quantize_once(size_t n, size_t bpr, int nmat);
 hipError_t launch_q4_gemv(const lgh_q4 *w0, float *y0, const lgh_q4 *w1, float *y1, const float *x,
                           int mode, int per_row, hipStream_t stream);
-// FFN gate/up stage of one decode token (lgh_ffn.hip): RMSNorm of x with
-// norm_w (null: none), ActQ8 (per_row mode) of the result, g = W1 normed and
-// u = W3 normed, h = silu(g) * u; writes the PerBlock ActQ8 codes hq [n] and
-// scales hs [n/32] of h when hq is not null, and h / g / u in f32 to hf / g /
-// u when those are not null.  W1, W3: n x k with n % 32 == 0, k <= 32 *
+// FFN gate/up stage of m <= kFfnMaxTokens tokens (lgh_ffn.hip): RMSNorm of the
+// rows x [m][k] with norm_w (null: none), ActQ8 (per_row mode) of the result,
+// g = W1 normed and u = W3 normed, h = silu(g) * u; writes the PerBlock ActQ8
+// codes hq [m][n] and scales hs [m][n/32] of h when hq is not null, and h / g /
+// u in f32 ([m][n]) to hf / g / u when those are not null.  W1, W3: n x k with n % 32 == 0, k <= 32 *
 // kFfnMaxBpr (one workgroup holds all of x's codes).
 constexpr size_t kFfnMaxBpr = 64;
+constexpr size_t kFfnMaxTokens = 4;
 bool ffn_gate_up_supported(const lgh_q4 *w1);
 hipError_t launch_ffn_gate_up(const lgh_q4 *w1, const lgh_q4 *w3, const float *x, const float *norm_w, float eps,
-                              int per_row, int8_t *hq, float *hs, float *hf, float *g, float *u,
+                              size_t m, int per_row, int8_t *hq, float *hs, float *hf, float *g, float *u,
                               hipStream_t stream);
 // rms_norm (ops.rs:8-23) over `rows` rows of `dim`, and g = silu(g) * u
 // (ops.rs:27-36, lfm2.rs:902-905); device pointers.
@@ -185,9 +186,13 @@ Q4BatchPlan plan_q4_batch(size_t m, size_t bpr);
 // Rows of > 64 blocks are quantized once (act_quant_kernel) and the kernel
 // reads the codes: inside it, every workgroup would quantize all m rows.
 bool q4_batch_quantize_once(size_t bpr);
-// codes / scales (ActQ8 of the m rows, [m][k] and [m][k/32]) replace x when non-null.
-hipError_t launch_q4_gemv_batch(const lgh_q4 *w, const float *x, const int8_t *codes, const float *scales, float *y,
-                                size_t m, int mode, int per_row, hipStream_t stream);
+// codes / scales (ActQ8 of the m rows, [m][k] and [m][k/32]) replace x when
+// non-null.  Up to three matrices with the same k in one launch; norm_w (not
+// null only where q4_batch_norms): rms_norm of the rows in the prologue.
+bool q4_batch_norms(size_t bpr);
+hipError_t launch_q4_gemv_batch(const lgh_q4 *const *w, float *const *y, int nmat, const float *x,
+                                const int8_t *codes, const float *scales, const float *norm_w, float eps, size_t m,
+                                int mode, int per_row, hipStream_t st);
 // Batched GEMV on the matrix cores for 2 <= m <= 64 (TT 16-token tiles, KW
 // K slices, CB-block chunks, RG 16-row groups per workgroup) on an
 // activation image written by act_quant_mma, with mt = ceil(m/16) token

@@ -1,0 +1,42 @@
+"""The FFN block of 2 to 4 tokens (two fused launches) equals the library's own op sequence bit for
+bit: every token slot count, rows that end inside a block group, a down projection whose kernel
+takes codes (inter 2080-8192), f32 rows (shorter) or the matrix-core batch route (longer), both
+act-quant modes, with and without the norm."""
+
+import numpy as np
+import pytest
+
+from llmhost_amd import q4, synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("per_row", [False, True])
+@pytest.mark.parametrize("norm", [True, False])
+@pytest.mark.parametrize("dim,inter,tokens", [(2048, 8192, 2), (1536, 8192, 3), (96, 2080, 4), (544, 2048, 2),
+                                              (1056, 64, 4), (2048, 10752, 3), (1536, 8224, 4)])
+def test_ffn_few_tokens_equals_op_sequence(gpu_ctx, dim, inter, tokens, norm, per_row):
+    shapes = ((inter, dim), (inter, dim), (dim, inter))
+    w1, w3, w2 = (q4.Q4Matrix.from_blocks(n, k, synth.q4_blocks(50 + i + n, n, k), gpu_ctx)
+                  for i, (n, k) in enumerate(shapes))
+    x = synth.activations(60 + tokens, tokens, dim)
+    x[tokens - 1, :32] = 0.0
+    nw = (1 + 0.1 * synth.normal_f32(61, dim)).astype(np.float32) if norm else None
+    q4.set_act_quant(q4.ActQuant.PerRow if per_row else q4.ActQuant.PerBlock, gpu_ctx)
+    try:
+        got = x.copy()
+        q4.ffn_residual(w1, w3, w2, nw, 1e-5, got, tokens)
+        normed = x.copy()
+        if norm:
+            q4.rms_norm(x, nw, 1e-5, normed, gpu_ctx)
+        g, u = (np.zeros((tokens, inter), dtype=np.float32) for _ in range(2))
+        q4.gemm_q4(w1, normed, g, tokens)
+        q4.gemm_q4(w3, normed, u, tokens)
+        q4.silu_mul(g, u, gpu_ctx)
+        ref = x.copy()
+        q4.gemm_q4_add(w2, g, ref, tokens)
+    finally:
+        q4.set_act_quant(q4.ActQuant.PerBlock, gpu_ctx)
+        for w in (w1, w3, w2):
+            w.free()
+    assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))

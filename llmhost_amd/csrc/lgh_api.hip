@@ -871,9 +871,9 @@ static int mma_chunked(lgh_ctx *ctx, const Ws &wsp, const lgh_q4 *const *w, int 
     else
       LGH_HIP(ctx, lgh::launch_act_quant_mma(x_dev + m0 * k, lgh::ActPrologue{}, mc, k, ctx->act_mode, ci, si,
                                              reinterpret_cast<float *>(ws + lay.o_rs), ctx->stream));
-    for (int j = 0; j < nmat; j++)
-      if (w[j]->n)
-        LGH_HIP(ctx, lgh::launch_q4_gemv_mma(w[j], ci, si, y_dev[j] + m0 * w[j]->n, mc, mode, ctx->stream, true));
+    float *yc[3] = {nullptr, nullptr, nullptr};
+    for (int j = 0; j < nmat; j++) yc[j] = w[j]->n ? y_dev[j] + m0 * w[j]->n : nullptr;
+    LGH_HIP(ctx, lgh::launch_q4_gemv_mma(w, yc, nmat, ci, si, mc, mode, ctx->stream, true));
   }
   return LGH_OK;
 }
@@ -960,8 +960,7 @@ static int gemm_multi_dev(lgh_ctx *ctx, const Ws &wsp, const lgh_q4 *const *w, i
     auto *si = reinterpret_cast<float *>(ws + o_si);
     LGH_HIP(ctx, lgh::launch_act_quant_mma(x_dev, pro, m, k, ctx->act_mode, ci, si,
                                            reinterpret_cast<float *>(ws + o_rs), ctx->stream));
-    for (int j = 0; j < nmat; j++)
-      if (w[j]->n) LGH_HIP(ctx, lgh::launch_q4_gemv_mma(w[j], ci, si, y_dev[j], m, mode, ctx->stream));
+    LGH_HIP(ctx, lgh::launch_q4_gemv_mma(w, y_dev, nmat, ci, si, m, mode, ctx->stream));
     return LGH_OK;
   }
   for (int j = 0; j < nmat; j++)

@@ -320,17 +320,19 @@ __global__ __launch_bounds__(W * kWave) void q4_gemv_batch_kernel(Q4BatchArgs a)
   const int lane = tid & (kWave - 1);
   const int wave = uniform(tid / kWave);
   const int rg = wave / KW, ks = wave % KW;
-  int wg = blockIdx.x, mat = 0;
+  int wg = blockIdx.x, n = a.n[0];
+  const uint8_t *qs = a.qs[0];
+  const uint16_t *sc = a.sc[0];
+  float *y = a.y[0];
   if (wg >= a.wgs0) {
     wg -= a.wgs0;
-    mat = 1;
-    if (wg >= a.wgs1) {
-      wg -= a.wgs1;
-      mat = 2;
-    }
+    const bool third = wg >= a.wgs1;
+    wg -= third ? a.wgs1 : 0;
+    n = third ? a.n[2] : a.n[1];
+    qs = third ? a.qs[2] : a.qs[1];
+    sc = third ? a.sc[2] : a.sc[1];
+    y = third ? a.y[2] : a.y[1];
   }
-  const int n = a.n[mat];
-  float *const y = a.y[mat];
   const int row0 = (wg * RG + rg) * 4;
   const int rows = uniform(max(0, min(4, n - row0)));
   const int r = lane >> 4, c = lane & 15;
@@ -377,8 +379,8 @@ __global__ __launch_bounds__(W * kWave) void q4_gemv_batch_kernel(Q4BatchArgs a)
 
   // (2) every weight load of this lane (rows past n read as 0).
   const size_t blk0 = static_cast<size_t>(row0) * bpr;
-  const auto wr = make_rsrc(a.qs[mat] + blk0 * 16, static_cast<uint32_t>(rows * bpr) * 16u);
-  const auto swr = make_rsrc(a.sc[mat] + blk0, static_cast<uint32_t>(rows * bpr) * 2u);
+  const auto wr = make_rsrc(qs + blk0 * 16, static_cast<uint32_t>(rows * bpr) * 16u);
+  const auto swr = make_rsrc(sc + blk0, static_cast<uint32_t>(rows * bpr) * 2u);
   uint4 w[BPL];
   uint16_t s[BPL];
 #pragma unroll
@@ -502,13 +504,29 @@ hipError_t launch_batch(Q4BatchArgs a, hipStream_t st) {
 // transposed to dwords through a per-wave LDS tile (row stride padded to
 // avoid bank conflicts); no workgroup barrier until the K-slice reduction.
 // Workgroup = 4 waves = RG row groups of 16 rows x KW K-slices.
-struct Q4MmaArgs {
+// Up to three matrices with the same k and plan share a launch (norm + q / k / v,
+// K=2048, 2048 + 2 x 512 rows, M = 8 / 24 / 40 / 64: 14.2 / 18.5 / 19.7 / 28.3 -> 7.7
+// / 9.4 / 10.1 / 13.2 us; the two short matrices alone fill 32 of 256 CUs):
+// workgroups [0, wgs0) cover matrix 0, the next wgs1 matrix 1, the rest matrix 2.
+struct MatRef {
   const uint8_t *qs;   // nibble plane [n][bpr][16]
   const uint16_t *sc;  // f16 scales [n][bpr]
+  float *y;            // [m][n]
+  int n;
+};
+
+// What a launch over one matrix reads fills the first 64 bytes, so that its
+// scalar loads go out together (a second round trip for ci and si cost 0.2 us of
+// M=64, K=2048, N=8192's 10.5).
+struct Q4MmaArgs {
+  const uint8_t *qs;   // matrix 0, as MatRef
+  const uint16_t *sc;
   const uint8_t *ci;   // activation codes image [mt][2 pq][64][16]
   const float *si;     // activation scales image [mt][pq][16][4]
-  float *y;            // [m][n]
+  float *y;
   int n, bpr, m, mode, mt, pq;
+  int wgs0, wgs1;
+  MatRef w1, w2;
 };
 
 typedef int v4i32 __attribute__((ext_vector_type(4)));
@@ -649,7 +667,7 @@ __device__ __forceinline__ void mma_compute(const MmaChunk<TT, CB> &c, uint32_t 
 // W = RG x KW waves: RG row groups of 16 rows, KW K slices.  The planner
 // gives each wave one chunk when the row allows it, so all of a wave's loads
 // are in flight at once (the GEMV's single round trip); longer rows loop.
-template <int TT, int KW, int CB, int RG, bool PF = false>
+template <int TT, int KW, int CB, int RG, bool PF, bool MULTI>
 __global__ __launch_bounds__(RG * KW * 64) void q4_mma_kernel(Q4MmaArgs a) {
   constexpr int W = RG * KW;
   constexpr int RS = CB * 4 + 4;
@@ -661,15 +679,27 @@ __global__ __launch_bounds__(RG * KW * 64) void q4_mma_kernel(Q4MmaArgs a) {
   const int lane = threadIdx.x & 63;
   const int wave = uniform(threadIdx.x >> 6);
   const int rg = wave / KW, ks = wave % KW;
-  const int row0 = (blockIdx.x * RG + rg) * 16;
-  const int rows = uniform(max(0, min(16, a.n - row0)));
+  int wg = blockIdx.x;
+  MatRef w{a.qs, a.sc, a.y, a.n};
+  if constexpr (MULTI) {
+    if (wg >= a.wgs0) {
+      wg -= a.wgs0;
+      w = a.w1;
+      if (wg >= a.wgs1) {
+        wg -= a.wgs1;
+        w = a.w2;
+      }
+    }
+  }
+  const int row0 = (wg * RG + rg) * 16;
+  const int rows = uniform(max(0, min(16, w.n - row0)));
   const int lr = lane & 15, g = lane >> 4;  // A: row lr; B / D: token lr; K group g
   const int nch = (bpr + CB - 1) / CB;
   const int ch_lo = nch * ks / KW, ch_hi = nch * (ks + 1) / KW;
 
   const size_t blk0 = static_cast<size_t>(row0) * bpr;
-  const auto wr = make_rsrc(a.qs + blk0 * 16, static_cast<uint32_t>(rows * bpr) * 16u);
-  const auto sr = make_rsrc(a.sc + blk0, static_cast<uint32_t>(rows * bpr) * 2u);
+  const auto wr = make_rsrc(w.qs + blk0 * 16, static_cast<uint32_t>(rows * bpr) * 16u);
+  const auto sr = make_rsrc(w.sc + blk0, static_cast<uint32_t>(rows * bpr) * 2u);
   const auto cr = make_rsrc(a.ci, static_cast<uint32_t>(a.mt * 2 * a.pq) * 1024u);
   const auto ar = make_rsrc(a.si, static_cast<uint32_t>(a.mt * a.pq) * 256u);
 
@@ -741,22 +771,32 @@ __global__ __launch_bounds__(RG * KW * 64) void q4_mma_kernel(Q4MmaArgs a) {
 #pragma unroll
     for (int v = 0; v < 4; v++) {
       const int r = 4 * g + v;
-      if (r < rows) store_row(a.y + static_cast<size_t>(t) * a.n, row0 + r, acc[tt][v], a.mode);
+      if (r < rows) store_row(w.y + static_cast<size_t>(t) * w.n, row0 + r, acc[tt][v], a.mode);
     }
   }
 }
 
 template <int TT, int KW, int CB, int RG>
-hipError_t launch_mma(const Q4MmaArgs &a, hipStream_t st) {
-  const int rows_per_wg = 16 * RG;
-  const unsigned wgs = static_cast<unsigned>((a.n + rows_per_wg - 1) / rows_per_wg);
+hipError_t launch_mma(Q4MmaArgs a, hipStream_t st) {
+  constexpr int kRows = 16 * RG;
+  a.wgs0 = (a.n + kRows - 1) / kRows;
+  a.wgs1 = (a.w1.n + kRows - 1) / kRows;
+  const unsigned wgs = static_cast<unsigned>(a.wgs0 + a.wgs1 + (a.w2.n + kRows - 1) / kRows);
+  const dim3 grid(wgs), blk(RG * KW * 64);
+  const bool multi = a.w1.n > 0;
   if constexpr (TT == 1 || TT == 4) {
     if ((a.bpr + CB - 1) / CB / KW >= 3) {  // every K slice has >= 3 chunks
-      hipLaunchKernelGGL((q4_mma_kernel<TT, KW, CB, RG, true>), dim3(wgs), dim3(RG * KW * 64), 0, st, a);
+      if (multi)
+        hipLaunchKernelGGL((q4_mma_kernel<TT, KW, CB, RG, true, true>), grid, blk, 0, st, a);
+      else
+        hipLaunchKernelGGL((q4_mma_kernel<TT, KW, CB, RG, true, false>), grid, blk, 0, st, a);
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((q4_mma_kernel<TT, KW, CB, RG>), dim3(wgs), dim3(RG * KW * 64), 0, st, a);
+  if (multi)
+    hipLaunchKernelGGL((q4_mma_kernel<TT, KW, CB, RG, false, true>), grid, blk, 0, st, a);
+  else
+    hipLaunchKernelGGL((q4_mma_kernel<TT, KW, CB, RG, false, false>), grid, blk, 0, st, a);
   return hipGetLastError();
 }
 
@@ -1206,12 +1246,47 @@ Q4MmaPlan plan_q4_mma(size_t n, size_t m, size_t bpr, bool any_shape) {
   return p;
 }
 
-hipError_t launch_q4_gemv_mma(const lgh_q4 *w, const uint8_t *codes, const float *scales, float *y, size_t m,
-                              int mode, hipStream_t st, bool any_shape) {
-  const Q4MmaPlan p = plan_q4_mma(w->n, m, w->bpr, any_shape);
-  if (!p.ok) return hipErrorInvalidValue;
-  Q4MmaArgs a{w->qs, w->sc, codes, scales, y, static_cast<int>(w->n), static_cast<int>(w->bpr), static_cast<int>(m),
-              mode, static_cast<int>((m + 15) / 16), static_cast<int>((w->bpr + 3) / 4)};
+hipError_t launch_q4_gemv_mma(const lgh_q4 *const *w, float *const *y, int nmat, const uint8_t *codes,
+                              const float *scales, size_t m, int mode, hipStream_t st, bool any_shape) {
+  if (nmat < 1 || nmat > 3) return hipErrorInvalidValue;
+  // A matrix's plan sets the order of its f32 additions, so it stays that of a
+  // launch of its own: matrices of one plan share a launch, the others follow.
+  Q4MmaPlan p{};
+  Q4MmaArgs a{};
+  MatRef mats[3] = {};
+  int rest = 0;
+  const lgh_q4 *rw[3];
+  float *ry[3];
+  int nj = 0;
+  for (int j = 0; j < nmat; j++) {
+    if (w[j]->n == 0) continue;
+    const Q4MmaPlan pj = plan_q4_mma(w[j]->n, m, w[j]->bpr, any_shape);
+    if (!pj.ok) return hipErrorInvalidValue;
+    if (nj == 0) p = pj;
+    if (pj.TT != p.TT || pj.KW != p.KW || pj.CB != p.CB || pj.RG != p.RG) {
+      rw[rest] = w[j];
+      ry[rest++] = y[j];
+      continue;
+    }
+    mats[nj++] = MatRef{w[j]->qs, w[j]->sc, y[j], static_cast<int>(w[j]->n)};
+  }
+  if (nj == 0) return hipSuccess;
+  if (rest) {
+    if (hipError_t e = launch_q4_gemv_mma(rw, ry, rest, codes, scales, m, mode, st, any_shape)) return e;
+  }
+  a.qs = mats[0].qs;
+  a.sc = mats[0].sc;
+  a.y = mats[0].y;
+  a.n = mats[0].n;
+  a.w1 = mats[1];
+  a.w2 = mats[2];
+  a.ci = codes;
+  a.si = scales;
+  a.bpr = static_cast<int>(w[0]->bpr);
+  a.m = static_cast<int>(m);
+  a.mode = mode;
+  a.mt = static_cast<int>((m + 15) / 16);
+  a.pq = static_cast<int>((w[0]->bpr + 3) / 4);
 #define LGH_M(TT_, KW_, CB_, RG_) \
   if (p.TT == TT_ && p.KW == KW_ && p.CB == CB_ && p.RG == RG_) return launch_mma<TT_, KW_, CB_, RG_>(a, st);
   LGH_MMA_SHAPES(LGH_M)

@@ -218,8 +218,9 @@ hipError_t launch_act_quant_mma(const float *x, ActPrologue pro, size_t m, size_
 // The same image from ActQ8 codes [m][k] and block scales [m][k/32].
 hipError_t launch_act_codes_mma(const int8_t *aq, const float *as, size_t m, size_t k, uint8_t *codes,
                                 float *scales, hipStream_t stream);
-hipError_t launch_q4_gemv_mma(const lgh_q4 *w, const uint8_t *codes, const float *scales, float *y, size_t m,
-                              int mode, hipStream_t stream, bool any_shape = false);
+// Up to three matrices with the same k; one launch for those of one plan.
+hipError_t launch_q4_gemv_mma(const lgh_q4 *const *w, float *const *y, int nmat, const uint8_t *codes,
+                              const float *scales, size_t m, int mode, hipStream_t stream, bool any_shape = false);
 // Q8_0 GEMV; K ranges of kQ8GemvMaxK (the Q4 GEMV plan's reach) and 65535
 // tokens per launch.  With norm_w not null (k <= kQ8GemvMaxK only) each
 // token's row is rms_norm'd in the prologue (eps as rms_norm).

@@ -379,19 +379,20 @@ __global__ __launch_bounds__(kThreads) void act_split_mx_kernel(const int8_t *__
 
 // Byte offset, in block b's pair record of token t's tile, of codes 4 g8 ..
 // 4 g8 + 3 of the block (MmaOrder, lgh_internal.h).
-__device__ __forceinline__ uint32_t mma_code_off(int t, int b, int g8, MmaOrder order) {
+template <MmaOrder Order>
+__device__ __forceinline__ uint32_t mma_code_off(int t, int b, int g8) {
   const uint32_t tok = t & 15;
-  return order == MmaOrder::kBlock ? (tok + 16 * (g8 >> 1)) * 16 + (b & 1) * 8 + (g8 & 1) * 4
+  return Order == MmaOrder::kBlock ? (tok + 16 * (g8 >> 1)) * 16 + (b & 1) * 8 + (g8 & 1) * 4
                                    : (tok + 16 * (2 * (b & 1) + (g8 >> 2))) * 16 + (g8 & 3) * 4;
 }
 
 // Activations for the matrix-core batch GEMV, in its MFMA register layouts
 // (lgh_internal.h): one 8-lane group per (token, block) over the padded
 // ranges [0, 16*mt) x [0, 4*pq); padding gets code 0 and scale 0.
+template <MmaOrder Order>
 __global__ __launch_bounds__(kThreads) void act_quant_mma_kernel(const float *__restrict__ x, ActPrologue pro, int m,
                                                                  int bpr, int pq, int per_row, const float *row_scale,
-                                                                 size_t groups, MmaOrder order, uint8_t *codes,
-                                                                 float *scales) {
+                                                                 size_t groups, uint8_t *codes, float *scales) {
   const size_t gi = (static_cast<size_t>(blockIdx.x) * kThreads + threadIdx.x) >> 3;
   if (gi >= groups) return;  // whole 8-lane groups exit together
   const int g8 = threadIdx.x & 7;
@@ -409,7 +410,7 @@ __global__ __launch_bounds__(kThreads) void act_quant_mma_kernel(const float *__
   int sum;
   const int q = act_quant_group8(v, pr, rs, scale, sum);
   const size_t pair = static_cast<size_t>(t >> 4) * (2 * pq) + (b >> 1);
-  *reinterpret_cast<int *>(codes + pair * 1024 + mma_code_off(t, b, g8, order)) = q;
+  *reinterpret_cast<int *>(codes + pair * 1024 + mma_code_off<Order>(t, b, g8)) = q;
   if (g8 == 0) scales[((static_cast<size_t>(t >> 4) * pq + (b >> 2)) * 16 + (t & 15)) * 4 + (b & 3)] = ok ? scale : 0.0f;
 }
 
@@ -447,12 +448,11 @@ __global__ __launch_bounds__(kThreads) void act_codes_mma_kernel(const int8_t *_
 // workgroup b takes token (b / 8) % TT of tile 8 (b / (8 TT)) + b % 8: the
 // rows of one tile, which share the image's cache lines, are written through
 // one XCD's L2.
-template <bool MX>
+template <bool MX, MmaOrder Order = MmaOrder::kBlock>
 __global__ __launch_bounds__(kThreads) void norm_image_kernel(const float *__restrict__ x,
                                                               const float *__restrict__ nw, double inv_k, float eps,
                                                               int m, int bpr, int nblk, int mt, int per_row,
-                                                              MmaOrder order, uint8_t *__restrict__ img,
-                                                              float *__restrict__ scales) {
+                                                              uint8_t *__restrict__ img, float *__restrict__ scales) {
   constexpr int TT = MX ? 32 : 16;
   constexpr int kRound = kThreads / 8;  // blocks per round of 8-lane groups
   constexpr int kPre = 4;               // rounds whose loads are in flight together
@@ -539,7 +539,7 @@ __global__ __launch_bounds__(kThreads) void norm_image_kernel(const float *__res
       } else {
         const int pq = nblk / 4;
         const size_t pair = static_cast<size_t>(tile) * (2 * pq) + (blk >> 1);
-        *reinterpret_cast<int *>(img + pair * 1024 + mma_code_off(t, blk, g8, order)) = q;
+        *reinterpret_cast<int *>(img + pair * 1024 + mma_code_off<Order>(t, blk, g8)) = q;
         if (g8 == 0)
           scales[((static_cast<size_t>(tile) * pq + (blk >> 2)) * 16 + (t & 15)) * 4 + (blk & 3)] = ok ? sc : 0.0f;
       }
@@ -547,15 +547,15 @@ __global__ __launch_bounds__(kThreads) void norm_image_kernel(const float *__res
   }
 }
 
-template <bool MX>
+template <bool MX, MmaOrder Order = MmaOrder::kBlock>
 hipError_t launch_norm_image(const float *x, const ActPrologue &pro, size_t m, size_t k, int per_row, int nblk,
-                             MmaOrder order, uint8_t *img, float *scales, hipStream_t st) {
+                             uint8_t *img, float *scales, hipStream_t st) {
   constexpr size_t TT = MX ? 32 : 16;
   const size_t mt = (m + TT - 1) / TT;
   const size_t wgs = (mt + 7) / 8 * 8 * TT;
-  hipLaunchKernelGGL(norm_image_kernel<MX>, dim3(static_cast<unsigned>(wgs)), dim3(kThreads), 0, st, x, pro.nw,
+  hipLaunchKernelGGL((norm_image_kernel<MX, Order>), dim3(static_cast<unsigned>(wgs)), dim3(kThreads), 0, st, x, pro.nw,
                      1.0 / static_cast<double>(k), pro.eps, static_cast<int>(m), static_cast<int>(k / 32), nblk,
-                     static_cast<int>(mt), per_row, order, img, scales);
+                     static_cast<int>(mt), per_row, img, scales);
   return hipGetLastError();
 }
 
@@ -589,8 +589,7 @@ hipError_t launch_act_quant_mx(const float *x, ActPrologue pro, size_t m, size_t
                                float *scratch, hipStream_t st) {
   const size_t bpr = k / 32, pp = (bpr + 1) / 2, mt = (m + 31) / 32;
   if (m == 0 || bpr == 0) return hipSuccess;
-  if (pro.nw) return launch_norm_image<true>(x, pro, m, k, per_row, static_cast<int>(2 * pp), MmaOrder::kBlock, mxa, nullptr,
-                                             st);
+  if (pro.nw) return launch_norm_image<true>(x, pro, m, k, per_row, static_cast<int>(2 * pp), mxa, nullptr, st);
   const float *rs = nullptr;
   if (hipError_t e = row_stats(x, pro, m, k, per_row, scratch, &rs, st)) return e;
   const size_t recs = mt * pp;  // < 2^31: the image is below kMxMaxBytes
@@ -604,14 +603,22 @@ hipError_t launch_act_quant_mma(const float *x, ActPrologue pro, size_t m, size_
                                 float *scales, float *scratch, hipStream_t st, MmaOrder order) {
   const size_t bpr = k / 32, pq = (bpr + 3) / 4, mt = (m + 15) / 16;
   if (m == 0 || bpr == 0) return hipSuccess;
+  const int nblk = static_cast<int>(4 * pq);
   if (pro.nw)
-    return launch_norm_image<false>(x, pro, m, k, per_row, static_cast<int>(4 * pq), order, codes, scales, st);
+    return order == MmaOrder::kBlock
+               ? launch_norm_image<false>(x, pro, m, k, per_row, nblk, codes, scales, st)
+               : launch_norm_image<false, MmaOrder::kPair>(x, pro, m, k, per_row, nblk, codes, scales, st);
   const float *rs = nullptr;
   if (hipError_t e = row_stats(x, pro, m, k, per_row, scratch, &rs, st)) return e;
   const size_t groups = mt * 16 * pq * 4;
-  hipLaunchKernelGGL(act_quant_mma_kernel, dim3(blocks_for(groups * 8, kThreads)), dim3(kThreads), 0, st, x, pro,
-                     static_cast<int>(m), static_cast<int>(bpr), static_cast<int>(pq), per_row, rs, groups, order,
-                     codes, scales);
+  const dim3 grid(blocks_for(groups * 8, kThreads)), blk(kThreads);
+  const int im = static_cast<int>(m), ib = static_cast<int>(bpr), iq = static_cast<int>(pq);
+  if (order == MmaOrder::kBlock)
+    hipLaunchKernelGGL(act_quant_mma_kernel<MmaOrder::kBlock>, grid, blk, 0, st, x, pro, im, ib, iq, per_row, rs,
+                       groups, codes, scales);
+  else
+    hipLaunchKernelGGL(act_quant_mma_kernel<MmaOrder::kPair>, grid, blk, 0, st, x, pro, im, ib, iq, per_row, rs,
+                       groups, codes, scales);
   return hipGetLastError();
 }
 

@@ -1,0 +1,27 @@
+"""Several matrices in one matrix-core batch launch (5 to 64 tokens) equal one launch each, bit for
+bit: matrices of one plan, a matrix whose own plan differs (three token tiles past 8192 rows), rows
+that end inside a 16-row tile, every number of token tiles."""
+
+import numpy as np
+import pytest
+
+from llmhost_amd import q4, synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("k,rows,tokens", [(2048, (2048, 512, 512), 40), (1568, (33, 1, 100), 5),
+                                           (1536, (8200, 256, 8192), 37), (1536, (64, 8208, 8224), 48),
+                                           (4096, (96, 130, 17), 64), (96, (48, 16), 17)])
+def test_norm_gemv_equals_one_matrix_at_a_time(gpu_ctx, k, rows, tokens):
+    ws = [q4.Q4Matrix.from_blocks(n, k, synth.q4_blocks(70 + i + n, n, k), gpu_ctx) for i, n in enumerate(rows)]
+    x = synth.activations(71 + tokens, tokens, k)
+    nw = (1 + 0.1 * synth.normal_f32(72, k)).astype(np.float32)
+    outs = [np.full((tokens, n), np.nan, dtype=np.float32) for n in rows]
+    q4.norm_gemv(ws, nw, 1e-5, x, outs, tokens)
+    for w, got in zip(ws, outs):
+        one = np.full_like(got, np.nan)
+        q4.norm_gemv([w], nw, 1e-5, x, [one], tokens)
+        assert np.array_equal(got.view(np.uint32), one.view(np.uint32))
+    for w in ws:
+        w.free()

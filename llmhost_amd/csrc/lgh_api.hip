@@ -1327,6 +1327,47 @@ static int ffn_fused(lgh_ctx *ctx, const lgh_q4 *w1, const lgh_q4 *w3, const lgh
   return LGH_OK;
 }
 
+// A prompt's FFN block with the gate/up GEMM writing the down projection's
+// operand image itself (*done: whether it applied).  Where both GEMMs run in
+// one token chunk, PerBlock, and the gate/up GEMM splits K nowhere; the values
+// are those of the general path.
+static int ffn_glu(lgh_ctx *ctx, const lgh_q4 *w1, const lgh_q4 *w3, const lgh_q4 *w2, const float *norm_w_dev,
+                   float eps, float *hidden_dev, size_t m, uint8_t *img, bool *done) {
+  *done = false;
+  const size_t dim = w1->k, inter = w1->n, mt = (m + 31) / 32;
+  const size_t rec_x = w1->pp * lgh::kMxARec, rec_h = w2->pp * lgh::kMxARec;
+  auto gemm = [&](const lgh_q4 *w) {  // m takes the GEMM route, in one chunk
+    return !lgh::plan_q4_batch(m, w->bpr).ok && !lgh::plan_q4_mma(w->n, m, w->bpr).ok && mx_fits(w) &&
+           mt + 8 <= lgh::kMxMaxBytes / (w->pp * lgh::kMxARec);
+  };
+  if (m < 2 || ctx->act_mode != LGH_ACT_PER_BLOCK || !gemm(w1) || !gemm(w3) || !gemm(w2) ||
+      !lgh::q4_glu_wanted(w1, w3, m))
+    return LGH_OK;
+  for (const lgh_q4 *w : {w1, w3, w2})
+    if (int r = ensure_mx(ctx, w)) return r;
+  // The workspace of the general path's two GEMM calls (its down projection's
+  // image region stays unused), so that a shape that ran once needs no growth
+  // in either act-quant mode.
+  const lgh::GemmPlan plan = lgh::plan_q4_gemm(&w2, 1, m);
+  const size_t part_floats = plan.splits > 1 ? static_cast<size_t>(plan.splits) * m * dim : 0;
+  Carve cv;
+  const size_t o_mx = cv.take(mt * std::max(rec_x, rec_h));
+  cv.take(m * sizeof(float));
+  const size_t o_part = cv.take(part_floats * sizeof(float));
+  char *ws = nullptr;
+  if (int r = grow_ws(ctx).get(cv.off, &ws)) return r;
+  auto *mxa = reinterpret_cast<uint8_t *>(ws + o_mx);
+  auto *part = reinterpret_cast<float *>(ws + o_part);
+  lgh::ActPrologue pro;
+  pro.nw = norm_w_dev;
+  pro.eps = eps;
+  LGH_HIP(ctx, lgh::launch_act_quant_mx(hidden_dev, pro, m, dim, 0, mxa, nullptr, ctx->stream));
+  LGH_HIP(ctx, lgh::launch_q4_glu(w1, w3, mxa, m, img, ctx->stream));
+  LGH_HIP(ctx, lgh::launch_q4_gemm(&w2, 1, img, &hidden_dev, m, LGH_ADD_F64, plan, part, part_floats, ctx->stream));
+  *done = inter > 0;
+  return LGH_OK;
+}
+
 int lgh_q4_ffn_residual_dev(lgh_ctx *ctx, const lgh_q4 *w1, const lgh_q4 *w3, const lgh_q4 *w2,
                             const float *norm_w_dev, float eps, float *hidden_dev, size_t tokens) {
   if (!ctx) return LGH_ERR_INVALID_ARG;
@@ -1350,6 +1391,11 @@ int lgh_q4_ffn_residual_dev(lgh_ctx *ctx, const lgh_q4 *w1, const lgh_q4 *w3, co
   if (int r = ensure(ctx, &ctx->ffn, &ctx->ffn_bytes, cv.off)) return r;
   char *f = static_cast<char *>(ctx->ffn);
   float *g = reinterpret_cast<float *>(f + o_g), *u = reinterpret_cast<float *>(f + o_u);
+  // The image of h (52 bytes per 32 elements) takes the place of g and u.
+  bool done = false;
+  if (int r = ffn_glu(ctx, w1, w3, w2, norm_w_dev, eps, hidden_dev, tokens, reinterpret_cast<uint8_t *>(g), &done))
+    return r;
+  if (done) return LGH_OK;
   const ActIn normed{hidden_dev, norm_w_dev, eps, nullptr, norm_w_dev ? reinterpret_cast<float *>(f + o_n) : nullptr};
   const lgh_q4 *gate_up[2] = {w1, w3};
   float *gu[2] = {g, u};

@@ -566,6 +566,29 @@ __device__ __forceinline__ void codes24_hl(int q4packed, uint32_t &vh, uint32_t 
   }
 }
 
+// The h / l E3M2 codes of every int8 code q, indexed by q + 128:
+// code(h) | code(l) << 6, read from this table into LDS by each workgroup
+// (a lookup in place of ~25 VALU per code).
+struct HlTable {
+  uint16_t v[256];
+};
+constexpr uint16_t e3m2_const(int v) {
+  int a = v < 0 ? -v : v, e = 0;
+  while ((2 << e) <= a) e++;
+  return static_cast<uint16_t>(a == 0 ? 0 : ((v < 0 ? 0x20 : 0) | ((e + 3) << 2) | (((a << 2) >> e) & 3)));
+}
+constexpr HlTable make_hl_table() {
+  HlTable t{};
+  for (int i = 0; i < 256; i++) {
+    const int q = i - 128, h = (q + 8) >> 4, l = q - 16 * h;  // split_h_l
+    t.v[i] = static_cast<uint16_t>(e3m2_const(h) | (e3m2_const(l) << 6));
+  }
+  return t;
+}
+static __constant__ HlTable kHlTable = make_hl_table();
+
+__device__ __forceinline__ uint16_t hl_table_entry(int i) { return kHlTable.v[i]; }
+
 // Byte offset of dword d (0..5) of operand row `row` within a 768-byte
 // (plane0 | plane1) tile image.
 __device__ __forceinline__ uint32_t mx_dword_off(int row, int d) {

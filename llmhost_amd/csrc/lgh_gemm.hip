@@ -72,6 +72,7 @@ struct Cfg {
   static constexpr int WL_W = W_CH / 64;                       // weight wave loads
   static constexpr int WL = WL_W + (A_CH + 63) / 64;           // all wave loads
   static constexpr int WPW = (WL + kThreads / 64 - 1) / (kThreads / 64);
+  static constexpr int W_STRIDE = kWRec;    // between a wave's weight tiles in a stage
   static constexpr int A_LDS = NS * kWRec;  // activation records start here in a stage
   static constexpr int STAGE = WPW * (kThreads / 64) * 1024;
   static_assert(WN * WM * 64 == kThreads, "4 waves per workgroup");
@@ -212,13 +213,13 @@ __device__ __forceinline__ void compute_stage(const char *buf, const StageOffs &
     float xs[TN], ys[TM];
     v8i A[2][TN], B[2][TM];
 #pragma unroll
-    for (int tn = 0; tn < TN; tn++) xs[tn] = *reinterpret_cast<const float *>(buf + o.ws + tn * kWRec);
+    for (int tn = 0; tn < TN; tn++) xs[tn] = *reinterpret_cast<const float *>(buf + o.ws + tn * C::W_STRIDE);
 #pragma unroll
     for (int tm = 0; tm < TM; tm++) ys[tm] = *reinterpret_cast<const float *>(buf + o.as + tm * kARec);
 #pragma unroll
     for (int b = 0; b < 2; b++) {
 #pragma unroll
-      for (int tn = 0; tn < TN; tn++) A[b][tn] = mx_operand(buf + o.a16[b] + tn * kWRec, buf + o.a8[b] + tn * kWRec);
+      for (int tn = 0; tn < TN; tn++) A[b][tn] = mx_operand(buf + o.a16[b] + tn * C::W_STRIDE, buf + o.a8[b] + tn * C::W_STRIDE);
 #pragma unroll
       for (int tm = 0; tm < TM; tm++) B[b][tm] = mx_operand(buf + o.b16[b] + tm * kARec, buf + o.b8[b] + tm * kARec);
     }
@@ -250,7 +251,7 @@ __device__ __forceinline__ void compute_stage(const char *buf, const StageOffs &
   float xs[TN], ys[TM];
   v8i A[2][TN], B[2][TM];
 #pragma unroll
-  for (int tn = 0; tn < TN; tn++) xs[tn] = *reinterpret_cast<const float *>(buf + o.ws + tn * kWRec);
+  for (int tn = 0; tn < TN; tn++) xs[tn] = *reinterpret_cast<const float *>(buf + o.ws + tn * C::W_STRIDE);
 #pragma unroll
   for (int tm = 0; tm < TM; tm++) ys[tm] = *reinterpret_cast<const float *>(buf + o.as + tm * kARec);
   v32f P[TN][TM];
@@ -261,7 +262,7 @@ __device__ __forceinline__ void compute_stage(const char *buf, const StageOffs &
 #pragma unroll
   for (int b = 0; b < 2; b++) {
 #pragma unroll
-    for (int tn = 0; tn < TN; tn++) A[b][tn] = mx_operand(buf + o.a16[b] + tn * kWRec, buf + o.a8[b] + tn * kWRec);
+    for (int tn = 0; tn < TN; tn++) A[b][tn] = mx_operand(buf + o.a16[b] + tn * C::W_STRIDE, buf + o.a8[b] + tn * C::W_STRIDE);
 #pragma unroll
     for (int tm = 0; tm < TM; tm++) B[b][tm] = mx_operand(buf + o.b16[b] + tm * kARec, buf + o.b8[b] + tm * kARec);
   }
@@ -452,6 +453,157 @@ __global__ __launch_bounds__(kThreads * KG) __attribute__((amdgpu_waves_per_eu(W
         }
       }
     }
+}
+
+// ---- gate / up GEMM with silu(g) * u and its activation image ---------------------
+// The FFN block's first GEMM and the launch between its two (h = silu(g) * u
+// and h's operand image) in one: a wave owns 32 rows of W1 and the same 32 rows
+// of W3 for 32 tokens (the wide launch's two 32 x 32 tiles, side by side in rows
+// instead of tokens), so g and u of an element meet in one lane, and a lane pair
+// (l, l + 32) holds a token's whole 32-element block of h.  It is quantized
+// there (act_quant's arithmetic) and stored as the block's h and l code rows
+// and scale: 512- and 256-byte runs.  g and u (8 bytes an element) are neither
+// written nor read back.
+// Workgroup = 2 x 2 waves: 64 rows of h (one block pair: one record per token
+// tile) x 64 tokens.  A stage holds W1's two records, W3's two, each pair
+// padded to 4 KB so that a wave load reads one matrix, then two activation
+// records: 15 wave loads, the 16 KB of the wide launch.
+struct GluCfg {
+  static constexpr int WPW = 4;
+  static constexpr int W_STRIDE = 4096;
+  static constexpr int A_LDS = 2 * W_STRIDE;
+  static constexpr int STAGE = 16384;
+};
+
+struct GluArgs {
+  GemmArgs g;          // W1's image, the activations'; n, m, nt, mt, pp
+  const uint8_t *w3x;  // W3's image
+  uint8_t *img;        // h's operand image [mt][pph]
+  int pph;             // block pairs of a row of h
+};
+
+__device__ __forceinline__ void glu_dma(const GluArgs &a, const Slots<GluCfg> &s, int wave, int p, int plive,
+                                        const char *buf) {
+  const i32x4 r1 = sgpr_rsrc(a.g.wmx, a.g.w_bytes), r3 = sgpr_rsrc(a.w3x, a.g.w_bytes);
+  const i32x4 ra = sgpr_rsrc(a.g.amx, a.g.a_bytes), rz = sgpr_rsrc(a.g.wmx, 0u);
+  const uint32_t base = lds_addr(buf);
+  const bool live = p < plive;  // as in dma_stage: a dead stage loads zeros
+  const int q = uniform(live ? p : 0);
+  const uint32_t sw = static_cast<uint32_t>(q * kWRec), sa = static_cast<uint32_t>(q * kARec);
+#pragma unroll
+  for (int i = 0; i < GluCfg::WPW; i++) {
+    const int j = wave + 4 * i;  // i = 0: W1, 1: W3, 2 and 3: activations
+    dma16(live ? (i == 0 ? r1 : i == 1 ? r3 : ra) : rz, s.off[i], i < 2 ? sw : sa,
+          base + 1024u * static_cast<uint32_t>(j));
+  }
+}
+
+template <int NB>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) void q4_glu_mx_kernel(GluArgs a) {
+  using C = GluCfg;
+  __shared__ __align__(1024) char lds[NB][C::STAGE];
+  __shared__ uint16_t s_hl[256];
+  const int wave = uniform(threadIdx.x >> 6), wn = wave & 1, wm = wave >> 1;
+  const int nt0 = blockIdx.x * 2, mt0 = blockIdx.y * 2;
+  const int lane = threadIdx.x & 63, tok = lane & 31, half = lane >> 5;
+  s_hl[threadIdx.x] = hl_table_entry(threadIdx.x);
+
+  float acc[2][1][16];
+#pragma unroll
+  for (int t = 0; t < 2; t++)
+#pragma unroll
+    for (int v = 0; v < 16; v++) acc[t][0][v] = 0.0f;
+
+  // Byte offsets of this lane's chunk in each wave load (stage 0), kOOB for
+  // padding; tiles past nt or mt land past their image and load as zeros.
+  Slots<C> slots;
+#pragma unroll
+  for (int i = 0; i < C::WPW; i++) {
+    const int c = 64 * (wave + 4 * (i < 2 ? 0 : i - 2)) + lane;
+    constexpr int kWCh = kWRec / 16, kACh = kARec / 16;
+    slots.off[i] = i < 2 ? (c < 2 * kWCh ? static_cast<uint32_t>((nt0 + c / kWCh) * a.g.pp) * kWRec + (c % kWCh) * 16
+                                         : kOOB)
+                         : (c < 2 * kACh ? static_cast<uint32_t>((mt0 + c / kACh) * a.g.pp) * kARec + (c % kACh) * 16
+                                         : kOOB);
+  }
+  const int wrec = wn * kWRec, arec = C::A_LDS + wm * kARec;
+  StageOffs o;
+#pragma unroll
+  for (int b = 0; b < 2; b++) {
+    o.a16[b] = opaque(wrec + b * kTile + tok * 16);
+    o.a8[b] = opaque(wrec + b * kTile + 512 + tok * 8);
+    o.b16[b] = opaque(arec + (2 * b + half) * kTile + tok * 16);
+    o.b8[b] = opaque(arec + (2 * b + half) * kTile + 512 + tok * 8);
+  }
+  o.ws = opaque(wrec + 2 * kTile + lane * 4);
+  o.as = opaque(arec + 4 * kTile + lane * 4);
+
+  const int pend = a.g.pp;
+  auto step = [&](int p, const char *cur, char *nxt) {  // pipeline_step
+    wait_vm_barrier<(NB - 2) * C::WPW>();
+    glu_dma(a, slots, wave, p + NB - 1, pend, nxt);
+    compute_stage<C, 2, 1>(cur, o, acc);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+#pragma unroll
+  for (int u = 0; u < NB - 1; u++) glu_dma(a, slots, wave, u, pend, lds[u]);
+  int p = 0;
+  for (; p + NB - 1 < pend; p += NB) {
+#pragma unroll
+    for (int u = 0; u < NB; u++) step(p + u, lds[u], lds[(u + NB - 1) % NB]);
+  }
+#pragma unroll
+  for (int u = 0; u < NB - 1; u++)
+    if (p + u < pend) step(p + u, lds[u], lds[(u + NB - 1) % NB]);
+  asm volatile("s_waitcnt vmcnt(0)" : : : "memory");  // as in q4_gemm_mx_kernel
+  if (a.g.pp < 1) __syncthreads();                    // the table, where no stage's barrier ordered it
+
+  // Lane: token tok, elements 8 q + 4 half + e of block nt0 + wn.  Tokens past
+  // m and rows past n have g = u = 0, h = 0: code 0, scale 0, the image's padding.
+  const int mt = mt0 + wm, pair = blockIdx.x;
+  if (mt >= a.g.mt) return;  // uniform
+  float h[16], mx = 0.0f;
+#pragma unroll
+  for (int v = 0; v < 16; v++) {
+    h[v] = silu_mul1(acc[0][0][v], acc[1][0][v]);
+    mx = fmaxf(mx, fabsf(h[v]));  // never NaN, as act_quant_group8's partials
+  }
+  const float amax = fmaxf(mx, __shfl_xor(mx, 32));
+  const float scale = div127_rn(amax);
+  const float inv = scale == 0.0f ? 0.0f : recip_rn(scale);
+  const float inv2 = 2.0f * inv;
+  const bool fast = inv2 <= 0x1.fffffep127f;
+  // Per 4 elements the 24-bit h and l streams; lane l + 0 builds the block's h
+  // row, lane l + 32 its l row, each from its own pieces and the partner's.
+  uint32_t mine[4], part[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    uint32_t vh = 0, vl = 0;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const float x = h[4 * q + e];
+      const int c = fast ? quant_code(x, inv2) : quant_code_ref(x, inv);
+      const uint32_t hl = s_hl[c + 128];
+      vh |= (hl & 63u) << (6 * e);
+      vl |= (hl >> 6) << (6 * e);
+    }
+    mine[q] = half ? vl : vh;
+    part[q] = static_cast<uint32_t>(__shfl_xor(static_cast<int>(half ? vh : vl), 32));
+  }
+  uint32_t d[6];
+#pragma unroll
+  for (int t = 0; t < 2; t++) {  // elements 16 t .. 16 t + 15: pieces 0 (half 0), 0 (half 1), 1, 1
+    const uint32_t p0 = half ? part[2 * t] : mine[2 * t], p1 = half ? mine[2 * t] : part[2 * t];
+    const uint32_t p2 = half ? part[2 * t + 1] : mine[2 * t + 1], p3 = half ? mine[2 * t + 1] : part[2 * t + 1];
+    d[3 * t] = p0 | (p1 << 24);
+    d[3 * t + 1] = (p1 >> 8) | (p2 << 16);
+    d[3 * t + 2] = (p2 >> 16) | (p3 << 8);
+  }
+  uint8_t *rec = a.img + (static_cast<size_t>(mt) * a.pph + pair) * kARec;
+  uint8_t *tile = rec + (2 * wn + half) * kTile;
+  *reinterpret_cast<uint4 *>(tile + tok * 16) = make_uint4(d[0], d[1], d[2], d[3]);
+  *reinterpret_cast<uint2 *>(tile + 512 + tok * 8) = make_uint2(d[4], d[5]);
+  if (half == 0) reinterpret_cast<float *>(rec + 4 * kTile)[wn * 32 + tok] = scale;
 }
 
 // Exact block dots through the same operand images and MFMA: one wave per
@@ -688,6 +840,39 @@ hipError_t launch_q4_gemm(const lgh_q4 *const *w, int nmat, const uint8_t *mxa, 
   // Otherwise 128 x 32 (4 waves, one 32 x 32 tile each, 108 VGPRs, 4 waves
   // per SIMD): the most workgroups resident to cover the stage loads.
   return launch_cfg<4, 1, 1, 1, 3, 4>(gm, nmat, splits, st);
+}
+
+// Without split K or K groups: those add an element's parts in another f32
+// order, and the block's results stay the general path's bits.  That leaves
+// launches of >= 512 128 x 32 tiles, where it won at every size measured
+// (figures above q4_glu_mx_kernel), down to 256 workgroups.
+bool q4_glu_wanted(const lgh_q4 *w1, const lgh_q4 *w3, size_t m) {
+  const lgh_q4 *w[2] = {w1, w3};
+  const GemmPlan plan = plan_q4_gemm(w, 2, m);
+  return plan.splits == 1 && plan.kgroups == 1 && w1->pp > 0;
+}
+
+hipError_t launch_q4_glu(const lgh_q4 *w1, const lgh_q4 *w3, const uint8_t *mxa, size_t m, uint8_t *img,
+                         hipStream_t st) {
+  if (m == 0 || w1->n == 0) return hipSuccess;
+  if (w1->n % 32 != 0 || w1->n != w3->n || w1->k != w3->k || w1->pp == 0) return hipErrorInvalidValue;
+  const size_t mt = (m + 31) / 32;
+  GluArgs a{};
+  a.g.wmx = w1->mx;
+  a.g.amx = mxa;
+  a.g.n = static_cast<int>(w1->n);
+  a.g.m = static_cast<int>(m);
+  a.g.nt = static_cast<int>(w1->nt);
+  a.g.mt = static_cast<int>(mt);
+  a.g.pp = static_cast<int>(w1->pp);
+  a.g.w_bytes = static_cast<uint32_t>(w1->nt * w1->pp * kMxWRec);
+  a.g.a_bytes = static_cast<uint32_t>(mt * w1->pp * kMxARec);
+  a.w3x = w3->mx;
+  a.img = img;
+  a.pph = static_cast<int>((w1->nt + 1) / 2);
+  const dim3 grid(static_cast<unsigned>(a.pph), static_cast<unsigned>((mt + 1) / 2));
+  hipLaunchKernelGGL(q4_glu_mx_kernel<3>, grid, dim3(kThreads), 0, st, a);
+  return hipGetLastError();
 }
 
 hipError_t launch_q4_mfma_block_dots(const lgh_q4 *w, const uint8_t *mxa, size_t m, int32_t *out,

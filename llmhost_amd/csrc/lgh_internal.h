@@ -256,6 +256,14 @@ GemmPlan plan_q4_gemm(const lgh_q4 *const *w, int nmat, size_t m);
 hipError_t launch_q4_gemm(const lgh_q4 *const *w, int nmat, const uint8_t *mxa, float *const *y, size_t m, int mode,
                           GemmPlan plan, float *part, size_t part_floats, hipStream_t stream);
 
+// Gate / up GEMM of the FFN block with h = silu(W1 x) * (W3 x) left as the
+// activation operand image of the down projection (PerBlock ActQ8), from the
+// image mxa of x: one launch, the values of launch_q4_gemm, silu_mul and
+// launch_act_quant_mx.  n % 32 == 0; img holds ceil(m/32) * ceil(n/64) records.
+bool q4_glu_wanted(const lgh_q4 *w1, const lgh_q4 *w3, size_t m);
+hipError_t launch_q4_glu(const lgh_q4 *w1, const lgh_q4 *w3, const uint8_t *mxa, size_t m, uint8_t *img,
+                         hipStream_t stream);
+
 // Measurement probes: an empty kernel of `wgs` workgroups, and a plain read
 // of `bytes` (a multiple of 16, 16-byte aligned) with per_thread (1, 2, 4, 8)
 // 16-byte loads per thread, one f32 sum per workgroup into out

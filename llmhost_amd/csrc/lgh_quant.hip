@@ -258,27 +258,6 @@ __device__ __forceinline__ void store_hl_group8(uint8_t *rec, int s, int tok, ui
   }
 }
 
-// The h / l E3M2 codes of every int8 code q, indexed by q + 128:
-// code(h) | code(l) << 6, read from this table into LDS by each workgroup
-// (a lookup in place of ~25 VALU per code).
-struct HlTable {
-  uint16_t v[256];
-};
-constexpr uint16_t e3m2_const(int v) {
-  int a = v < 0 ? -v : v, e = 0;
-  while ((2 << e) <= a) e++;
-  return static_cast<uint16_t>(a == 0 ? 0 : ((v < 0 ? 0x20 : 0) | ((e + 3) << 2) | (((a << 2) >> e) & 3)));
-}
-constexpr HlTable make_hl_table() {
-  HlTable t{};
-  for (int i = 0; i < 256; i++) {
-    const int q = i - 128, h = (q + 8) >> 4, l = q - 16 * h;  // split_h_l
-    t.v[i] = static_cast<uint16_t>(e3m2_const(h) | (e3m2_const(l) << 6));
-  }
-  return t;
-}
-__constant__ HlTable kHlTable = make_hl_table();
-
 // Activations -> the GEMM's operand image, one record (r = token tile * pp +
 // block pair: 32 tokens x 2 blocks) per workgroup.  The 64 four-lane groups
 // each quantize one (token, block): group G = tid / 4 takes token G % 32 of
@@ -312,7 +291,7 @@ __global__ __launch_bounds__(kThreads) void act_quant_mx_kernel(const float *__r
     apply_prologue(pro, f, a);
     apply_prologue(pro, f + 1, b);
   }
-  s_hl[tid] = kHlTable.v[tid];
+  s_hl[tid] = hl_table_entry(tid);
   __syncthreads();  // the table
   const bool pr = ok && per_row;
   const float rs = pr ? row_scale[t] : 0.0f;

@@ -235,6 +235,9 @@ bool q8_batch_wanted(const lgh_q8 *w, size_t tokens);
 hipError_t launch_q8_mma(const lgh_q8 *w, const uint8_t *codes, const float *scales, float *y, size_t m,
                          hipStream_t stream);
 
+// words 4-byte words from src to dst (either may be pinned host memory).
+hipError_t launch_copy_words(const void *src, void *dst, size_t words, hipStream_t stream);
+
 // Batched activation quantization: x[m][k] -> qs[m][k], scales[m][k/32]
 // (+ sums if non-null).  row_scale: scratch of m floats (used for per_row).
 hipError_t launch_act_quant(const float *x, size_t m, size_t k, int per_row, int8_t *qs,

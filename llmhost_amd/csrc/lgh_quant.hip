@@ -70,6 +70,15 @@ __global__ __launch_bounds__(kThreads) void act_quant_kernel(const float *__rest
   }
 }
 
+// A small host call's operands between pinned host memory and the device: one
+// 4-byte word a thread, so the row lengths need no alignment; a wave's 256 bytes
+// are one PCIe burst either way.
+__global__ __launch_bounds__(kThreads) void copy_words_kernel(const uint32_t *__restrict__ src,
+                                                              uint32_t *__restrict__ dst, size_t words) {
+  const size_t i = static_cast<size_t>(blockIdx.x) * kThreads + threadIdx.x;
+  if (i < words) dst[i] = src[i];
+}
+
 // ---- load-time kernels ----------------------------------------------------
 // Raw BlockQ4 (18 bytes) -> repacked nibble block + f16 scale.
 __device__ __forceinline__ uint32_t raw_nib(const uint8_t *q, int e) {
@@ -682,6 +691,13 @@ hipError_t launch_act_quant(const float *x, size_t m, size_t k, int per_row, int
   const size_t threads = m * bpr * 8;
   hipLaunchKernelGGL(act_quant_kernel, dim3(blocks_for(threads, kThreads)), dim3(kThreads), 0, st, x,
                      static_cast<int>(m), static_cast<int>(bpr), per_row, row_scale, qs, scales, sums);
+  return hipGetLastError();
+}
+
+hipError_t launch_copy_words(const void *src, void *dst, size_t words, hipStream_t st) {
+  if (words == 0) return hipSuccess;
+  hipLaunchKernelGGL(copy_words_kernel, dim3(blocks_for(words, kThreads)), dim3(kThreads), 0, st,
+                     static_cast<const uint32_t *>(src), static_cast<uint32_t *>(dst), words);
   return hipGetLastError();
 }
 

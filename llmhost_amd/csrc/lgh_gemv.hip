@@ -1146,9 +1146,13 @@ hipError_t launch_q4_gemv_multi(const lgh_q4 *const *w, float *const *y, int nma
   return hipErrorInvalidValue;
 }
 
-// m <= 4 tokens in T = 4 slots; K: one slice of BPL <= 4 blocks per lane up
-// to 64 blocks, then 2 or 4 slices of 64 (the prologue quantizes 4 rows of
-// up to 8192 elements).  Other shapes run the matrix-core batch kernel.
+// m <= 4 tokens in T = 4 slots; K: one slice of BPL <= 4 blocks per lane up to
+// 64 blocks, then 2 or 4 slices of 64, and 8 of 48 or 64 up to 512 blocks (the
+// codes of 4 rows of 16384 elements are 72 KB of LDS: two workgroups a CU).
+// Against the matrix-core batch kernel, which longer rows run, the whole call
+// at M = 4: K=10752, N=2048 / 8192 / 10752 13.0 / 21.4 / 28.0 -> 9.6 / 20.8 / 25.8
+// us; K=16384, N=512 / 8192 15.9 / 30.6 -> 8.6 / 25.8 us; M = 2 alike; the FFN
+// block of dim 2048, inter 10752 28.1 -> 22.4 us (its down projection takes codes).
 Q4BatchPlan plan_q4_batch(size_t m, size_t bpr) {
   Q4BatchPlan p{};
   if (m < 2 || m > 4 || bpr == 0) return p;
@@ -1158,6 +1162,9 @@ Q4BatchPlan plan_q4_batch(size_t m, size_t bpr) {
   } else if (bpr <= 256) {
     p.KW = bpr <= 128 ? 2 : 4;
     p.BPL = 4;
+  } else if (bpr <= 512) {
+    p.KW = 8;
+    p.BPL = bpr <= 384 ? 3 : 4;
   } else {
     return p;
   }
@@ -1201,6 +1208,7 @@ hipError_t launch_q4_gemv_batch(const lgh_q4 *const *w, float *const *y, int nma
   a.per_row = per_row;
   if (codes) {
     if (p.KW == 1) return hipErrorInvalidValue;
+    if (p.KW == 8) return p.BPL == 3 ? launch_batch<3, 8, true>(a, st) : launch_batch<4, 8, true>(a, st);
     return p.KW == 2 ? launch_batch<4, 2, true>(a, st) : launch_batch<4, 4, true>(a, st);
   }
   if (p.KW == 1) {

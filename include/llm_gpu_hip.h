@@ -302,9 +302,9 @@ int lgh_silu_mul_dev(lgh_ctx *ctx, float *g_dev, const float *u_dev, size_t n);
  * Otherwise the ops above run on the device one after another, except that
  * for 5 or more tokens the norm and the gate/up activation image are
  * formed in one launch (the normed rows are not written) and silu(g) * u in
- * the launch that writes the down projection's image -- on the GEMM route,
- * PerBlock and without split K, the gate/up GEMM itself; the results equal
- * the op sequence's bit for bit.
+ * the launch that writes the down projection's image -- PerBlock, for up to 32
+ * tokens and on the GEMM route without split K, the gate/up launch itself; the
+ * results equal the op sequence's bit for bit.
  * No single reference function: it replaces the reference's sequence of
  * calls. */
 int lgh_q4_ffn_residual(lgh_ctx *ctx, const lgh_q4 *w1, const lgh_q4 *w3, const lgh_q4 *w2,

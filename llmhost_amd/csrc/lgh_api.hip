@@ -1407,6 +1407,36 @@ static int ffn_fused(lgh_ctx *ctx, const lgh_q4 *w1, const lgh_q4 *w3, const lgh
   return LGH_OK;
 }
 
+// The FFN block of 5 to 32 tokens with the gate/up launch writing the down
+// projection's activation image (*done: whether it applied); PerBlock, both
+// projections on the matrix-core batch route.  The values are those of the
+// general path.
+static int ffn_mma_glu(lgh_ctx *ctx, const lgh_q4 *w1, const lgh_q4 *w3, const lgh_q4 *w2, const float *norm_w_dev,
+                       float eps, float *hidden_dev, size_t m, uint8_t *img, bool *done) {
+  *done = false;
+  // inter >= 128: the image of up to 15 padding tokens fits where g and u were.
+  if (m < 5 || ctx->act_mode != LGH_ACT_PER_BLOCK || w1->n < 128 || !lgh::q4_mma_glu_wanted(w1, m) ||
+      !lgh::plan_q4_mma(w2->n, m, w2->bpr).ok)
+    return LGH_OK;
+  const size_t mt = (m + 15) / 16, pq = (w1->bpr + 3) / 4, pqh = (w2->bpr + 3) / 4;
+  Carve cv;  // as the general path's two calls (ffn_glu)
+  const size_t o_ci = cv.take(mt * std::max(pq, pqh) * 2 * 1024), o_si = cv.take(mt * std::max(pq, pqh) * 256);
+  cv.take(m * sizeof(float));
+  char *ws = nullptr;
+  if (int r = grow_ws(ctx).get(cv.off, &ws)) return r;
+  auto *ci = reinterpret_cast<uint8_t *>(ws + o_ci);
+  auto *si = reinterpret_cast<float *>(ws + o_si);
+  auto *so = reinterpret_cast<float *>(img + mt * pqh * 2 * 1024);
+  lgh::ActPrologue pro;
+  pro.nw = norm_w_dev;
+  pro.eps = eps;
+  LGH_HIP(ctx, lgh::launch_act_quant_mma(hidden_dev, pro, m, w1->k, 0, ci, si, nullptr, ctx->stream));
+  LGH_HIP(ctx, lgh::launch_q4_mma_glu(w1, w3, ci, si, m, img, so, ctx->stream));
+  LGH_HIP(ctx, lgh::launch_q4_gemv_mma(&w2, &hidden_dev, 1, img, so, m, LGH_ADD_F64, ctx->stream));
+  *done = true;
+  return LGH_OK;
+}
+
 // A prompt's FFN block with the gate/up GEMM writing the down projection's
 // operand image itself (*done: whether it applied).  Where both GEMMs run in
 // one token chunk, PerBlock, and the gate/up GEMM splits K nowhere; the values
@@ -1474,6 +1504,9 @@ int lgh_q4_ffn_residual_dev(lgh_ctx *ctx, const lgh_q4 *w1, const lgh_q4 *w3, co
   // The image of h (52 bytes per 32 elements) takes the place of g and u.
   bool done = false;
   if (int r = ffn_glu(ctx, w1, w3, w2, norm_w_dev, eps, hidden_dev, tokens, reinterpret_cast<uint8_t *>(g), &done))
+    return r;
+  if (done) return LGH_OK;
+  if (int r = ffn_mma_glu(ctx, w1, w3, w2, norm_w_dev, eps, hidden_dev, tokens, reinterpret_cast<uint8_t *>(g), &done))
     return r;
   if (done) return LGH_OK;
   const ActIn normed{hidden_dev, norm_w_dev, eps, nullptr, norm_w_dev ? reinterpret_cast<float *>(f + o_n) : nullptr};

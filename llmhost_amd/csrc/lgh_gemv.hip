@@ -776,6 +776,115 @@ __global__ __launch_bounds__(RG * KW * 64) void q4_mma_kernel(Q4MmaArgs a) {
   }
 }
 
+// ---- gate / up of the FFN block on the matrix cores, with silu and the codes -------
+// The FFN block of 5 to 32 tokens: h = silu(W1 x) * (W3 x) and h's activation
+// image in one launch.  A workgroup is one 32-row block of h: 2 x 16 rows x 8 K
+// slices, a wave holding the same 16 rows of W1 and W3 (so the activation
+// operands are loaded once for both), each with q4_mma_kernel's chunk loop and
+// slice sums; g and u of an element then meet in one lane, h in LDS, and 8
+// lanes a token quantize the block into the image (act_quant_mma_kernel's
+// arithmetic and layout).
+struct MmaGluArgs {
+  Q4MmaArgs a;          // W1 (qs, sc), the image of x; n, bpr, m, mt, pq
+  const uint8_t *qs3;   // W3
+  const uint16_t *sc3;
+  uint8_t *co;          // h's image: codes, scales, block quads per row
+  float *so;
+  int pqo;
+};
+
+template <int TT>
+__global__ __launch_bounds__(1024) void q4_mma_glu_kernel(MmaGluArgs ga) {
+  constexpr int CB = 8, KW = 8, W = 2 * KW, RS = CB * 4 + 4;
+  constexpr int kWords = W * 16 * RS, kScales = W * CB * 16, kPart = W * 2 * TT * 4 * 64;
+  // The weights' transpose tiles, then (behind a barrier) the slices' sums.
+  __shared__ __align__(16) uint32_t s_mem[kWords + kScales > kPart ? kWords + kScales : kPart];
+  __shared__ __align__(16) float s_h[TT * 16][36];
+  const Q4MmaArgs &a = ga.a;
+  const int bpr = a.bpr;
+  const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
+  const int rt = wave / KW, ks = wave % KW;
+  const int row0 = blockIdx.x * 32 + rt * 16;  // n % 32 == 0: every row exists
+  const int lr = lane & 15, g = lane >> 4;
+  const int nch = (bpr + CB - 1) / CB;
+  const int ch_lo = nch * ks / KW, ch_hi = nch * (ks + 1) / KW;
+  const size_t blk0 = static_cast<size_t>(row0) * bpr;
+  const uint32_t wb = static_cast<uint32_t>(16 * bpr) * 16u, sb = static_cast<uint32_t>(16 * bpr) * 2u;
+  const auto wr1 = make_rsrc(a.qs + blk0 * 16, wb), wr3 = make_rsrc(ga.qs3 + blk0 * 16, wb);
+  const auto sr1 = make_rsrc(a.sc + blk0, sb), sr3 = make_rsrc(ga.sc3 + blk0, sb);
+  const auto cr = make_rsrc(a.ci, static_cast<uint32_t>(a.mt * 2 * a.pq) * 1024u);
+  const auto ar = make_rsrc(a.si, static_cast<uint32_t>(a.mt * a.pq) * 256u);
+
+  float acc[2][TT][4];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int tt = 0; tt < TT; tt++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) acc[i][tt][v] = 0.0f;
+  uint32_t *tw = s_mem + wave * 16 * RS;
+  float *tsw = reinterpret_cast<float *>(s_mem + kWords) + wave * CB * 16;
+  for (int ch = ch_lo; ch < ch_hi; ch++) {
+    MmaChunk<TT, CB> c1, c3;
+    mma_load<TT, CB, 1>(a, wr1, sr1, cr, ar, ch, c1);
+    mma_load<TT, CB, 1>(a, wr3, sr3, cr, ar, ch, c3);
+    mma_load<TT, CB, 2>(a, wr1, sr1, cr, ar, ch, c1);
+#pragma unroll
+    for (int tt = 0; tt < TT; tt++) {
+#pragma unroll
+      for (int j = 0; j < CB / 2; j++) c3.bq[tt][j] = c1.bq[tt][j];
+#pragma unroll
+      for (int j = 0; j < CB / 4; j++) c3.sa[tt][j] = c1.sa[tt][j];
+    }
+    mma_compute<TT, CB>(c1, tw, tsw, acc[0]);
+    mma_compute<TT, CB>(c3, tw, tsw, acc[1]);
+  }
+  __syncthreads();  // every wave is done with its tiles
+  float *part = reinterpret_cast<float *>(s_mem);
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int tt = 0; tt < TT; tt++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) part[((wave * 2 + i) * TT * 4 + tt * 4 + v) * 64 + lane] = acc[i][tt][v];
+  __syncthreads();
+  // Wave w < 2 TT: rows 16 (w / TT) + 4 g + v of token 16 (w % TT) + lr, the slices in order.
+  if (wave < 2 * TT) {
+    const int r2 = wave / TT, tt = wave % TT;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      float gu[2];
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        float sum = 0.0f;
+#pragma unroll
+        for (int k = 0; k < KW; k++) sum += part[(((r2 * KW + k) * 2 + i) * TT * 4 + tt * 4 + v) * 64 + lane];
+        gu[i] = sum * 0.0625f;  // exact: undo the x16 of the unpack
+      }
+      s_h[tt * 16 + lr][r2 * 16 + 4 * g + v] = silu_mul1(gu[0], gu[1]);
+    }
+  }
+  __syncthreads();
+  // Token t by 8 lanes; tokens past m have h = 0: code 0, scale 0.  The last
+  // workgroup also clears the blocks that pad the row to a quad.
+  const int t = threadIdx.x >> 3, g8 = threadIdx.x & 7;
+  if (t >= TT * 16) return;
+  auto put = [&](int blk, int q, float scale) {
+    const size_t pair = static_cast<size_t>(t >> 4) * (2 * ga.pqo) + (blk >> 1);
+    const int ln = (t & 15) + 16 * (g8 >> 1);
+    *reinterpret_cast<int *>(ga.co + (pair * 64 + ln) * 16 + (blk & 1) * 8 + (g8 & 1) * 4) = q;
+    if (g8 == 0)
+      ga.so[((static_cast<size_t>(t >> 4) * ga.pqo + (blk >> 2)) * 16 + (t & 15)) * 4 + (blk & 3)] = scale;
+  };
+  const int blk = blockIdx.x, nblk = gridDim.x;
+  float scale;
+  int sum;
+  const int q = act_quant_group8(*reinterpret_cast<const float4 *>(&s_h[t][4 * g8]), false, 0.0f, scale, sum);
+  put(blk, q, scale);
+  if (blk == nblk - 1)
+    for (int b = nblk; b < 4 * ga.pqo; b++) put(b, 0, 0.0f);
+}
+
 template <int TT, int KW, int CB, int RG>
 hipError_t launch_mma(Q4MmaArgs a, hipStream_t st) {
   constexpr int kRows = 16 * RG;
@@ -1300,6 +1409,40 @@ hipError_t launch_q4_gemv_mma(const lgh_q4 *const *w, float *const *y, int nmat,
   LGH_MMA_SHAPES(LGH_M)
 #undef LGH_M
   return hipErrorInvalidValue;
+}
+
+// The gate/up launch keeps q4_mma_kernel's sums, so it stands in for plans of one
+// or two token tiles in 8-block chunks over 8 K slices (33 to 192 blocks a row).
+bool q4_mma_glu_wanted(const lgh_q4 *w1, size_t m) {
+  const Q4MmaPlan p = plan_q4_mma(w1->n, m, w1->bpr);
+  return p.ok && p.TT <= 2 && p.KW == 8 && p.CB == 8 && w1->n % 32 == 0 && (p.TT == 2 || w1->bpr <= 192);
+}
+
+hipError_t launch_q4_mma_glu(const lgh_q4 *w1, const lgh_q4 *w3, const uint8_t *codes, const float *scales, size_t m,
+                             uint8_t *codes_out, float *scales_out, hipStream_t st) {
+  if (m == 0 || w1->n == 0) return hipSuccess;
+  if (!q4_mma_glu_wanted(w1, m) || w3->n != w1->n || w3->k != w1->k) return hipErrorInvalidValue;
+  MmaGluArgs ga{};
+  ga.a.qs = w1->qs;
+  ga.a.sc = w1->sc;
+  ga.a.ci = codes;
+  ga.a.si = scales;
+  ga.a.n = static_cast<int>(w1->n);
+  ga.a.bpr = static_cast<int>(w1->bpr);
+  ga.a.m = static_cast<int>(m);
+  ga.a.mt = static_cast<int>((m + 15) / 16);
+  ga.a.pq = static_cast<int>((w1->bpr + 3) / 4);
+  ga.qs3 = w3->qs;
+  ga.sc3 = w3->sc;
+  ga.co = codes_out;
+  ga.so = scales_out;
+  const int nblk = static_cast<int>(w1->n / 32);
+  ga.pqo = (nblk + 3) / 4;
+  if (ga.a.mt == 1)
+    hipLaunchKernelGGL(q4_mma_glu_kernel<1>, dim3(nblk), dim3(1024), 0, st, ga);
+  else
+    hipLaunchKernelGGL(q4_mma_glu_kernel<2>, dim3(nblk), dim3(1024), 0, st, ga);
+  return hipGetLastError();
 }
 
 hipError_t launch_q8_range(const lgh_q8 *w, const float *x, float *y, size_t tokens, const float *norm_w, float eps,

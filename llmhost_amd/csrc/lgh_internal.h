@@ -221,6 +221,13 @@ hipError_t launch_act_codes_mma(const int8_t *aq, const float *as, size_t m, siz
 // Up to three matrices with the same k; one launch for those of one plan.
 hipError_t launch_q4_gemv_mma(const lgh_q4 *const *w, float *const *y, int nmat, const uint8_t *codes,
                               const float *scales, size_t m, int mode, hipStream_t stream, bool any_shape = false);
+// Gate / up of the FFN block for the tokens and rows that q4_mma_glu_wanted
+// accepts: h = silu(W1 x) * (W3 x) as the down projection's image (kBlock,
+// PerBlock), from the image of x; the values of launch_q4_gemv_mma and
+// launch_act_quant_mma.
+bool q4_mma_glu_wanted(const lgh_q4 *w1, size_t m);
+hipError_t launch_q4_mma_glu(const lgh_q4 *w1, const lgh_q4 *w3, const uint8_t *codes, const float *scales, size_t m,
+                             uint8_t *codes_out, float *scales_out, hipStream_t stream);
 // Q8_0 GEMV; K ranges of kQ8GemvMaxK (the Q4 GEMV plan's reach) and 65535
 // tokens per launch.  With norm_w not null (k <= kQ8GemvMaxK only) each
 // token's row is rms_norm'd in the prologue (eps as rms_norm).

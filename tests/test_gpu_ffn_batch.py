@@ -1,7 +1,8 @@
-"""The FFN block of 2 to 4 tokens (two fused launches) equals the library's own op sequence bit for
+"""The FFN block of 2 to 32 tokens (two or three fused launches) equals the library's own op sequence bit for
 bit: every token slot count, rows that end inside a block group, a down projection whose kernel
-takes codes (inter 2080-8192), f32 rows (shorter) or the matrix-core batch route (longer), both
-act-quant modes, with and without the norm."""
+takes codes (inter 2080-8192), f32 rows (shorter) or the matrix-core batch route (longer); from 5
+tokens on, one and two token tiles, block counts of h that pad its image's quad by 0 to 3, rows of
+33 to 65 blocks and one more slice chunk; both act-quant modes, with and without the norm."""
 
 import numpy as np
 import pytest
@@ -14,7 +15,9 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("per_row", [False, True])
 @pytest.mark.parametrize("norm", [True, False])
 @pytest.mark.parametrize("dim,inter,tokens", [(2048, 8192, 2), (1536, 8192, 3), (96, 2080, 4), (544, 2048, 2),
-                                              (1056, 64, 4), (2048, 10752, 3), (1536, 8224, 4)])
+                                              (1056, 64, 4), (2048, 10752, 3), (1536, 8224, 4),
+                                              (1536, 8192, 13), (1056, 128, 5), (2048, 160, 16), (2080, 192, 17),
+                                              (1568, 2272, 32), (4128, 256, 9)])
 def test_ffn_few_tokens_equals_op_sequence(gpu_ctx, dim, inter, tokens, norm, per_row):
     shapes = ((inter, dim), (inter, dim), (dim, inter))
     w1, w3, w2 = (q4.Q4Matrix.from_blocks(n, k, synth.q4_blocks(50 + i + n, n, k), gpu_ctx)

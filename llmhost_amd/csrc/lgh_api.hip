@@ -64,6 +64,15 @@ int set_device(lgh_ctx *ctx) {
   return LGH_OK;
 }
 
+// Set a workspace that a captured call uses aside instead of letting it be freed.
+void keep_captured(lgh_ctx *ctx) {
+  if (!ctx->ws_captured || !ctx->ws) return;
+  ctx->kept.push_back(ctx->ws);
+  ctx->ws = nullptr;
+  ctx->ws_bytes = 0;
+  ctx->ws_captured = false;
+}
+
 // Grow-only device buffer; waits for queued work before releasing the old one.
 // A stream under graph capture cannot synchronize or allocate: growing there
 // fails with LGH_ERR_CAPTURE (the caller warms the shape up eagerly first, or
@@ -76,6 +85,7 @@ int ensure(lgh_ctx *ctx, void **buf, size_t *cap, size_t bytes) {
                 "a workspace must grow to %zu bytes while the stream is being captured; run the same "
                 "shape once before capturing, or call lgh_q4_gemm_dev_noalloc",
                 bytes);
+  if (buf == &ctx->ws) keep_captured(ctx);
   if (*buf) {
     LGH_HIP(ctx, hipStreamSynchronize(ctx->stream));
     LGH_HIP(ctx, hipFree(*buf));
@@ -372,6 +382,7 @@ void lgh_destroy(lgh_ctx *ctx) {
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
   if (ctx->ws) (void)hipFree(ctx->ws);
+  for (void *p : ctx->kept) (void)hipFree(p);
   if (ctx->stage) (void)hipFree(ctx->stage);
   if (ctx->ffn) (void)hipFree(ctx->ffn);
   if (ctx->own_stream) (void)hipStreamDestroy(ctx->own_stream);
@@ -417,6 +428,7 @@ int lgh_trim(lgh_ctx *ctx) {
   if (!ctx) return LGH_ERR_INVALID_ARG;
   if (int r = set_device(ctx)) return r;
   LGH_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  keep_captured(ctx);
   release(ctx, &ctx->ws, &ctx->ws_bytes);
   release(ctx, &ctx->stage, &ctx->stage_bytes);
   release(ctx, &ctx->ffn, &ctx->ffn_bytes);
@@ -1151,7 +1163,9 @@ static bool capturing(lgh_ctx *ctx) {
 // The Q8_0 product of `tokens` rows of x, rms_norm'd first when nw is not null.
 // Several tokens of a large matrix: up to 64 at a time, their activation image
 // (with the norm) and one pass over the weights.  Otherwise, and where
-// the image's workspace would have to grow under capture, the GEMV.
+// the image's workspace would have to grow under capture, the GEMV.  A graph of
+// the pass stays good when later calls grow the workspace (keep_captured), as
+// one of the GEMV, which has no workspace, does.
 static int q8_rows(lgh_ctx *ctx, const lgh_q8 *w, const float *x, const float *nw, float eps, float *y,
                    size_t tokens) {
   const size_t k = w->k, pq = (w->bpr + 3) / 4;
@@ -1159,9 +1173,11 @@ static int q8_rows(lgh_ctx *ctx, const lgh_q8 *w, const float *x, const float *n
   const size_t passes = (tokens + 63) / 64, mt = ((tokens + passes - 1) / passes + 15) / 16, chunk = mt * 16;
   Carve cv;
   const size_t o_ci = cv.take(mt * pq * 2 * 1024), o_si = cv.take(mt * pq * 256);
-  if (lgh::q8_batch_wanted(w, tokens) && (cv.off <= ctx->ws_bytes || !capturing(ctx))) {
+  const bool wanted = lgh::q8_batch_wanted(w, tokens), captured = wanted && capturing(ctx);
+  if (wanted && (cv.off <= ctx->ws_bytes || !captured)) {
     char *ws = nullptr;
     if (int r = grow_ws(ctx).get(cv.off, &ws)) return r;
+    ctx->ws_captured = ctx->ws_captured || captured;
     auto *ci = reinterpret_cast<uint8_t *>(ws + o_ci);
     auto *si = reinterpret_cast<float *>(ws + o_si);
     lgh::ActPrologue pro;

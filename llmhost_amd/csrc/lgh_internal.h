@@ -36,6 +36,7 @@
 #include <cstdint>
 #include <mutex>
 #include <string>
+#include <vector>
 
 #include "../../include/llm_gpu_hip.h"
 
@@ -49,6 +50,10 @@ struct lgh_ctx {
   // GEMM workspace: activation operand image, f32 row scales [m], split-K partials.
   void *ws = nullptr;
   size_t ws_bytes = 0;
+  // A captured Q8_0 call holds the workspace's address: growing or trimming it
+  // then keeps the old buffer in `kept`, until the context goes.
+  bool ws_captured = false;
+  std::vector<void *> kept;
   // Device staging for the host-pointer entry points.
   void *stage = nullptr;
   size_t stage_bytes = 0;

@@ -75,3 +75,45 @@ def test_q8_batch_under_capture_without_a_workspace(oracle):
     del graph
     w.free()
     ctx.close()
+
+
+def test_q8_batch_graph_survives_growth_and_trim(oracle):
+    """A captured pass keeps its workspace when a later call grows it and when it is trimmed."""
+    import torch
+
+    n, k, tokens = 8192, 2048, 16
+    blocks = synth.q8_blocks(5, n, k)
+    ctx = q4.Context(0)
+    stream = torch.cuda.Stream()
+    ctx.set_stream(stream.cuda_stream)
+    w = q4.Q8Matrix.from_blocks(n, k, blocks, ctx)
+    w4 = q4.Q4Matrix.from_blocks(64, 8192, synth.q4_blocks(6, 64, 8192), ctx)
+    xh = synth.activations(6, tokens, k)
+    x = torch.from_numpy(xh).cuda()
+    y = torch.zeros(tokens, n, device="cuda")
+    x4, y4 = torch.randn(600, 8192, device="cuda"), torch.zeros(600, 64, device="cuda")
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        q4.q8_apply(w, x, tokens, y)  # sizes the workspace
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            q4.q8_apply(w, x, tokens, y)
+    ref = oracle.q8_apply(blocks, n, k, xh, tokens, threads=8).reshape(tokens, n)
+    for step in range(3):
+        with torch.cuda.stream(stream):
+            if step == 1:
+                q4.gemm_q4(w4, x4, y4, 600)
+            if step == 2:
+                ctx.trim()
+            junk = torch.full((1 << 22,), float("nan"), device="cuda")  # what was freed is written over
+            y.zero_()
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+        assert_close(y.cpu().numpy(), ref, what=f"replay {step}")
+        del junk
+    del graph
+    w.free()
+    w4.free()
+    ctx.close()

@@ -422,8 +422,8 @@ __global__ __launch_bounds__(kThreads) void act_codes_mma_kernel(const int8_t *_
 }
 
 // ---- rms_norm in the activation images ---------------------------------------
-// rms_norm (ops.rs:8-23) and an activation image in one launch, one
-// workgroup per token row of the padded token range.  The sum of squares is
+// rms_norm (ops.rs:8-23; without NORM nothing, for the PerRow scale alone) and an
+// activation image in one launch, one workgroup per token row of the padded token range.  The sum of squares is
 // formed exactly as rms_norm_kernel forms it (thread i adds the f64 squares
 // of elements i, i + 256, ... in turn; DPP wave trees; the 4 wave sums in
 // order), so the scale and every normed value nw * (x * scale) equal the op
@@ -436,7 +436,7 @@ __global__ __launch_bounds__(kThreads) void act_codes_mma_kernel(const int8_t *_
 // workgroup b takes token (b / 8) % TT of tile 8 (b / (8 TT)) + b % 8: the
 // rows of one tile, which share the image's cache lines, are written through
 // one XCD's L2.
-template <bool MX, MmaOrder Order = MmaOrder::kBlock>
+template <bool MX, MmaOrder Order = MmaOrder::kBlock, bool NORM = true>
 __global__ __launch_bounds__(kThreads) void norm_image_kernel(const float *__restrict__ x,
                                                               const float *__restrict__ nw, double inv_k, float eps,
                                                               int m, int bpr, int nblk, int mt, int per_row,
@@ -453,51 +453,56 @@ __global__ __launch_bounds__(kThreads) void norm_image_kernel(const float *__res
   const uint32_t row_bytes = static_cast<uint32_t>(k) * 4u;
   // Rows past m read as zeros (a resource of size 0) and are stored as zeros.
   const auto xr = make_rsrc(x + static_cast<size_t>(live ? t : 0) * k, live ? row_bytes : 0u);
-  const auto nr = make_rsrc(nw, row_bytes);
+  const auto nr = make_rsrc(nw, NORM ? row_bytes : 0u);
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
   const int g8 = tid & 7, grp = tid >> 3;
   // The first rounds' float4s of x and nw (blocks past bpr read 0), requested
   // before the sum of squares so they arrive while it is formed.
-  float4 xa[kPre], wa[kPre];
+  float4 xa[kPre], wa[NORM ? kPre : 1];
   auto load_rounds = [&](int b0) {
 #pragma unroll
     for (int u = 0; u < kPre; u++) {
       const uint32_t off = static_cast<uint32_t>((b0 + kRound * u + grp) * 8 + g8) * 16u;
       xa[u] = buf_load_f4(xr, off);
-      wa[u] = buf_load_f4(nr, off);
+      if constexpr (NORM) wa[u] = buf_load_f4(nr, off);
     }
   };
   load_rounds(0);
-  // Thread i: the squares of elements i, i + 256, ... in order, 8 loads in
-  // flight; elements past k read 0 and add +0.0, which changes no sum.
-  double ss = 0.0;
-  for (int i0 = 0; i0 < k; i0 += kThreads * 8) {
-    float v[8];
-#pragma unroll
-    for (int u = 0; u < 8; u++) v[u] = buf_load_f32(xr, static_cast<uint32_t>(i0 + tid + kThreads * u) * 4u);
-#pragma unroll
-    for (int u = 0; u < 8; u++) {
-      const double d = v[u];
-      ss += d * d;
-    }
-  }
   __shared__ double s_ss[kWaves];
   __shared__ float s_mx[kWaves];
-  ss = wave_sum_dpp64(ss);
-  if (lane == 0) s_ss[wave] = ss;
-  __syncthreads();
-  double tot = 0.0;
+  float scale = 1.0f;
+  if constexpr (NORM) {
+    // Thread i: the squares of elements i, i + 256, ... in order, 8 loads in
+    // flight; elements past k read 0 and add +0.0, which changes no sum.
+    double ss = 0.0;
+    for (int i0 = 0; i0 < k; i0 += kThreads * 8) {
+      float v[8];
 #pragma unroll
-  for (int i = 0; i < kWaves; i++) tot += s_ss[i];
-  const float scale = rms_scale(tot, inv_k, eps);
+      for (int u = 0; u < 8; u++) v[u] = buf_load_f32(xr, static_cast<uint32_t>(i0 + tid + kThreads * u) * 4u);
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        const double d = v[u];
+        ss += d * d;
+      }
+    }
+    ss = wave_sum_dpp64(ss);
+    if (lane == 0) s_ss[wave] = ss;
+    __syncthreads();
+    double tot = 0.0;
+#pragma unroll
+    for (int i = 0; i < kWaves; i++) tot += s_ss[i];
+    scale = rms_scale(tot, inv_k, eps);
+  }
   float rs = 0.0f;
   if (per_row) {  // amax(nw * (x * scale)) / 127, as row_amax_kernel over the normed rows
     float mx = 0.0f;
     for (int f = tid; f < k / 4; f += kThreads) {
-      const float4 a = buf_load_f4(xr, static_cast<uint32_t>(f) * 16u);
-      const float4 w = buf_load_f4(nr, static_cast<uint32_t>(f) * 16u);
-      mx = fmaxf(mx, fmaxf(fmaxf(fabsf(w.x * (a.x * scale)), fabsf(w.y * (a.y * scale))),
-                           fmaxf(fabsf(w.z * (a.z * scale)), fabsf(w.w * (a.w * scale)))));
+      float4 a = buf_load_f4(xr, static_cast<uint32_t>(f) * 16u);
+      if constexpr (NORM) {
+        const float4 w = buf_load_f4(nr, static_cast<uint32_t>(f) * 16u);
+        a = make_float4(w.x * (a.x * scale), w.y * (a.y * scale), w.z * (a.z * scale), w.w * (a.w * scale));
+      }
+      mx = fmaxf(mx, fmaxf(fmaxf(fabsf(a.x), fabsf(a.y)), fmaxf(fabsf(a.z), fabsf(a.w))));
     }
     mx = wave_max(mx);
     if (lane == 0) s_mx[wave] = mx;
@@ -510,10 +515,14 @@ __global__ __launch_bounds__(kThreads) void norm_image_kernel(const float *__res
     for (int u = 0; u < kPre; u++) {
       const int blk = b0 + kRound * u + grp;
       const bool ok = live && blk < bpr;
-      const float4 a = xa[u], w = wa[u];
-      const float4 v = ok ? make_float4(w.x * (a.x * scale), w.y * (a.y * scale), w.z * (a.z * scale),
-                                        w.w * (a.w * scale))
-                          : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      if (ok) {
+        v = xa[u];
+        if constexpr (NORM) {
+          const float4 w = wa[u];
+          v = make_float4(w.x * (v.x * scale), w.y * (v.y * scale), w.z * (v.z * scale), w.w * (v.w * scale));
+        }
+      }
       float sc;
       int sum;
       const int q = act_quant_group8(v, ok && per_row, rs, sc, sum);
@@ -535,13 +544,13 @@ __global__ __launch_bounds__(kThreads) void norm_image_kernel(const float *__res
   }
 }
 
-template <bool MX, MmaOrder Order = MmaOrder::kBlock>
+template <bool MX, MmaOrder Order = MmaOrder::kBlock, bool NORM = true>
 hipError_t launch_norm_image(const float *x, const ActPrologue &pro, size_t m, size_t k, int per_row, int nblk,
                              uint8_t *img, float *scales, hipStream_t st) {
   constexpr size_t TT = MX ? 32 : 16;
   const size_t mt = (m + TT - 1) / TT;
   const size_t wgs = (mt + 7) / 8 * 8 * TT;
-  hipLaunchKernelGGL((norm_image_kernel<MX, Order>), dim3(static_cast<unsigned>(wgs)), dim3(kThreads), 0, st, x, pro.nw,
+  hipLaunchKernelGGL((norm_image_kernel<MX, Order, NORM>), dim3(static_cast<unsigned>(wgs)), dim3(kThreads), 0, st, x, pro.nw,
                      1.0 / static_cast<double>(k), pro.eps, static_cast<int>(m), static_cast<int>(k / 32), nblk,
                      static_cast<int>(mt), per_row, img, scales);
   return hipGetLastError();
@@ -562,6 +571,19 @@ hipError_t launch_q4_mx_pack(const lgh_q4 *w, hipStream_t st) {
   return hipGetLastError();
 }
 
+// PerRow images whose row scale is formed by the workgroup that holds the row
+// (norm_image_kernel without the norm) instead of a launch before the image's.
+// Whole calls, two launches against one: K=2048, N=2048, M = 8 / 128 10.0 / 16.2 ->
+// 9.6 / 15.1 us; K=2048, N=8192, M = 16 / 40 / 97 11.5 / 15.0 / 18.9 -> 10.2 / 13.6 /
+// 17.7; K=4096, N=2048, M=64 (8192 blocks) 16.6 -> 15.3.  Its partial-line stores
+// lose on many blocks (K=2048, M=777, 49728: 7.6 us against 4.0 + 4.8, the call
+// among others 56.8 -> 58.4; K=N=2048, M=2048 19.8 -> 21.0), and rows longer than the
+// 128 blocks whose loads are in flight together are read twice (K=8192, M=64 12.5
+// -> 14.2; K=10752, M=200 18.0 -> 20.7).
+bool row_image_wanted(const ActPrologue &pro, size_t m, size_t bpr, int per_row) {
+  return per_row && !pro.u && bpr <= 128 && m * bpr <= 8192;
+}
+
 // The PerRow scale an image kernel needs before it starts (row_amax_kernel
 // over x or silu(x) * u).  scratch: m floats.
 hipError_t row_stats(const float *x, const ActPrologue &pro, size_t m, size_t k, int per_row, float *scratch,
@@ -578,6 +600,9 @@ hipError_t launch_act_quant_mx(const float *x, ActPrologue pro, size_t m, size_t
   const size_t bpr = k / 32, pp = (bpr + 1) / 2, mt = (m + 31) / 32;
   if (m == 0 || bpr == 0) return hipSuccess;
   if (pro.nw) return launch_norm_image<true>(x, pro, m, k, per_row, static_cast<int>(2 * pp), mxa, nullptr, st);
+  if (row_image_wanted(pro, m, bpr, per_row))
+    return launch_norm_image<true, MmaOrder::kBlock, false>(x, pro, m, k, 1, static_cast<int>(2 * pp), mxa, nullptr,
+                                                            st);
   const float *rs = nullptr;
   if (hipError_t e = row_stats(x, pro, m, k, per_row, scratch, &rs, st)) return e;
   const size_t recs = mt * pp;  // < 2^31: the image is below kMxMaxBytes
@@ -596,6 +621,8 @@ hipError_t launch_act_quant_mma(const float *x, ActPrologue pro, size_t m, size_
     return order == MmaOrder::kBlock
                ? launch_norm_image<false>(x, pro, m, k, per_row, nblk, codes, scales, st)
                : launch_norm_image<false, MmaOrder::kPair>(x, pro, m, k, per_row, nblk, codes, scales, st);
+  if (row_image_wanted(pro, m, bpr, per_row))  // kPair images are PerBlock
+    return launch_norm_image<false, MmaOrder::kBlock, false>(x, pro, m, k, 1, nblk, codes, scales, st);
   const float *rs = nullptr;
   if (hipError_t e = row_stats(x, pro, m, k, per_row, scratch, &rs, st)) return e;
   const size_t groups = mt * 16 * pq * 4;

@@ -1320,15 +1320,13 @@ hipError_t launch_q4_gemv_batch(const lgh_q4 *const *w, float *const *y, int nma
     if (p.KW == 8) return p.BPL == 3 ? launch_batch<3, 8, true>(a, st) : launch_batch<4, 8, true>(a, st);
     return p.KW == 2 ? launch_batch<4, 2, true>(a, st) : launch_batch<4, 4, true>(a, st);
   }
-  if (p.KW == 1) {
-    switch (p.BPL) {
-      case 1: return launch_batch<1, 1>(a, st);
-      case 2: return launch_batch<2, 1>(a, st);
-      case 3: return launch_batch<3, 1>(a, st);
-      default: return launch_batch<4, 1>(a, st);
-    }
+  if (p.KW != 1) return hipErrorInvalidValue;  // q4_batch_quantize_once
+  switch (p.BPL) {
+    case 1: return launch_batch<1, 1>(a, st);
+    case 2: return launch_batch<2, 1>(a, st);
+    case 3: return launch_batch<3, 1>(a, st);
+    default: return launch_batch<4, 1>(a, st);
   }
-  return p.KW == 2 ? launch_batch<4, 2>(a, st) : launch_batch<4, 4>(a, st);
 }
 
 // Token tiles TT = ceil(m / 16) (<= 4); 8-block chunks; KW (a power of

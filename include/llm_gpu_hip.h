@@ -94,7 +94,9 @@ int lgh_sync(lgh_ctx *ctx);
  * buffers (GEMM workspace, host-call staging, FFN intermediates); they grow
  * again on the next call that needs them.  Workspaces grow only outside
  * stream capture: a call under capture that would grow one returns
- * LGH_ERR_CAPTURE, so run each shape once before capturing.  No reference
+ * LGH_ERR_CAPTURE, so run each shape once before capturing.  (A workspace that
+ * a captured Q8_0 call of several tokens uses is kept until lgh_destroy
+ * instead, also when a later call grows it.)  No reference
  * counterpart (llm-cpu keeps no device buffers). */
 int lgh_trim(lgh_ctx *ctx);
 

@@ -1,7 +1,7 @@
-"""Two to four tokens over rows of 257 to 512 blocks (8 K slices in a workgroup) against the
-exact value (64-bit sums of the oracle's codes), at the edges: one block past 8192 elements, the last row length of 3 blocks per lane and
-one more, 16384 elements and one block past them (the matrix-core route), rows that leave lanes
-idle, both act-quant modes and an addition."""
+"""Two to four tokens over rows of 257 to 512 blocks (8 K slices in a workgroup) against the exact
+value (64-bit sums of the oracle's codes), at the edges: one block past 8192 elements, the last row
+length of 3 blocks per lane and one more, 16384 elements and one block past them (the matrix-core
+route), rows that leave lanes idle, both act-quant modes and an addition."""
 
 import numpy as np
 import pytest

@@ -91,12 +91,16 @@ void *lgh_get_stream(const lgh_ctx *ctx);
 /* Wait for all work enqueued on the context stream. */
 int lgh_sync(lgh_ctx *ctx);
 /* Wait for the context stream, then release the context's grow-only device
- * buffers (GEMM workspace, host-call staging, FFN intermediates); they grow
- * again on the next call that needs them.  Workspaces grow only outside
+ * buffers (GEMM workspace, host-call staging, FFN intermediates, the Q8_0
+ * calls' activation image); they grow again on the next call that needs them.
+ * Workspaces grow only outside
  * stream capture: a call under capture that would grow one returns
- * LGH_ERR_CAPTURE, so run each shape once before capturing.  (A workspace that
- * a captured Q8_0 call of several tokens uses is kept until lgh_destroy
- * instead, also when a later call grows it.)  No reference
+ * LGH_ERR_CAPTURE, so run each shape once before capturing.  A graph keeps the
+ * addresses of the workspaces its calls were captured with: it is good until a
+ * later call grows one of them, lgh_trim or lgh_destroy; and as graphs and
+ * eager calls of one context write the same workspaces, the caller orders them
+ * (one stream, or events between streams).  Neither holds for Q8_0 calls, which
+ * use none when captured (lgh_q8_gemv).  No reference
  * counterpart (llm-cpu keeps no device buffers). */
 int lgh_trim(lgh_ctx *ctx);
 
@@ -259,9 +263,14 @@ int lgh_probe_read_dev(lgh_ctx *ctx, const void *src_dev, size_t bytes, int per_
  * with per-block ActQ8 activations.  Assign mode only, as in the reference.
  * Any K and any number of tokens (rows past 32768 elements are summed in
  * K ranges of 32768, added in f32).  Several tokens of a large matrix share
- * one pass over the weights per 64 tokens, on an activation image in the
- * context's workspace (a captured call that would have to grow it reads the
- * weights once per token instead). */
+ * one pass over the weights per 64 tokens, on an activation image: eager calls
+ * share one of the context, a captured call gets one of its own from the matrix,
+ * so that its graph needs the matrix, x and y only -- it may be replayed on any
+ * stream, beside other calls, and after lgh_destroy.  A matrix holds the images
+ * of captured calls until lgh_q8_free, up to 64 MiB; a call past that, as one
+ * without device memory for its image, reads the weights once per token.  The
+ * f32 summation order, and so the last bits of a row, differ between the two
+ * ways: between one token and several, as on the Q4 routes. */
 int lgh_q8_gemv(lgh_ctx *ctx, const lgh_q8 *w, const float *x, float *y, size_t tokens);
 int lgh_q8_gemv_dev(lgh_ctx *ctx, const lgh_q8 *w, const float *x_dev, float *y_dev,
                     size_t tokens);

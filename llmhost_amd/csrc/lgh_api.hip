@@ -64,15 +64,6 @@ int set_device(lgh_ctx *ctx) {
   return LGH_OK;
 }
 
-// Set a workspace that a captured call uses aside instead of letting it be freed.
-void keep_captured(lgh_ctx *ctx) {
-  if (!ctx->ws_captured || !ctx->ws) return;
-  ctx->kept.push_back(ctx->ws);
-  ctx->ws = nullptr;
-  ctx->ws_bytes = 0;
-  ctx->ws_captured = false;
-}
-
 // Grow-only device buffer; waits for queued work before releasing the old one.
 // A stream under graph capture cannot synchronize or allocate: growing there
 // fails with LGH_ERR_CAPTURE (the caller warms the shape up eagerly first, or
@@ -85,7 +76,6 @@ int ensure(lgh_ctx *ctx, void **buf, size_t *cap, size_t bytes) {
                 "a workspace must grow to %zu bytes while the stream is being captured; run the same "
                 "shape once before capturing, or call lgh_q4_gemm_dev_noalloc",
                 bytes);
-  if (buf == &ctx->ws) keep_captured(ctx);
   if (*buf) {
     LGH_HIP(ctx, hipStreamSynchronize(ctx->stream));
     LGH_HIP(ctx, hipFree(*buf));
@@ -234,7 +224,13 @@ int alloc_matrix(lgh_ctx *ctx, size_t n, size_t k, size_t qs_bytes_per_block, M 
   return LGH_OK;
 }
 
-void free_extra(lgh_q8 *) {}
+void free_extra(lgh_q8 *w) {
+  while (lgh_q8::Image *i = w->images) {
+    w->images = i->next;
+    (void)hipFree(i->p);
+    delete i;
+  }
+}
 void free_extra(lgh_q4 *w) {
   if (w->mx) (void)hipFree(w->mx);
 }
@@ -382,7 +378,7 @@ void lgh_destroy(lgh_ctx *ctx) {
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
   if (ctx->ws) (void)hipFree(ctx->ws);
-  for (void *p : ctx->kept) (void)hipFree(p);
+  if (ctx->q8_img) (void)hipFree(ctx->q8_img);
   if (ctx->stage) (void)hipFree(ctx->stage);
   if (ctx->ffn) (void)hipFree(ctx->ffn);
   if (ctx->own_stream) (void)hipStreamDestroy(ctx->own_stream);
@@ -428,8 +424,8 @@ int lgh_trim(lgh_ctx *ctx) {
   if (!ctx) return LGH_ERR_INVALID_ARG;
   if (int r = set_device(ctx)) return r;
   LGH_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  keep_captured(ctx);
   release(ctx, &ctx->ws, &ctx->ws_bytes);
+  release(ctx, &ctx->q8_img, &ctx->q8_img_bytes);
   release(ctx, &ctx->stage, &ctx->stage_bytes);
   release(ctx, &ctx->ffn, &ctx->ffn_bytes);
   return LGH_OK;
@@ -1160,39 +1156,83 @@ static bool capturing(lgh_ctx *ctx) {
   return hipStreamIsCapturing(ctx->stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
 }
 
+// Allocations while this thread's or another thread's stream is being captured:
+// none of them becomes a node of the graph.
+struct AllocUnderCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  AllocUnderCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~AllocUnderCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+// What the images of one matrix's captured calls may hold: about 450 calls of
+// 64 tokens at K=2048.
+constexpr size_t kQ8CapturedBytes = size_t(64) << 20;
+
+// Activation image of a Q8_0 pass, `bytes` for the call and `full` for 64 tokens
+// of its rows; null where there is none (the caller then takes the GEMV, which
+// needs none).  Eager calls of a context are ordered by its stream and share one
+// buffer, of the full size so that it grows only for longer rows.  A captured
+// call gets a buffer of its own, which nothing else ever uses: its graph may be
+// replayed on any stream, beside other calls and graphs, and after the context
+// is gone.  It belongs to the matrix, without which the graph is not good either.
+static char *q8_image(lgh_ctx *ctx, const lgh_q8 *wc, size_t bytes, size_t full) {
+  AllocUnderCapture relaxed;
+  if (!capturing(ctx)) {
+    if (full <= ctx->q8_img_bytes || ensure(ctx, &ctx->q8_img, &ctx->q8_img_bytes, full) == LGH_OK)
+      return static_cast<char *>(ctx->q8_img);
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  auto *w = const_cast<lgh_q8 *>(wc);
+  std::lock_guard<std::mutex> lock(w->images_mu);
+  const size_t want = align_up(bytes);
+  if (w->images_bytes + want > kQ8CapturedBytes) return nullptr;
+  auto *img = new (std::nothrow) lgh_q8::Image();
+  if (!img) return nullptr;
+  if (hipMalloc(&img->p, want) != hipSuccess) {
+    (void)hipGetLastError();
+    delete img;
+    return nullptr;
+  }
+  img->next = w->images;
+  w->images = img;
+  w->images_bytes += want;
+  return static_cast<char *>(img->p);
+}
+
 // The Q8_0 product of `tokens` rows of x, rms_norm'd first when nw is not null.
 // Several tokens of a large matrix: up to 64 at a time, their activation image
-// (with the norm) and one pass over the weights.  Otherwise, and where
-// the image's workspace would have to grow under capture, the GEMV.  A graph of
-// the pass stays good when later calls grow the workspace (keep_captured), as
-// one of the GEMV, which has no workspace, does.
+// (with the norm) and one pass over the weights.  Otherwise, and where there is
+// no memory for the image, the GEMV.
 static int q8_rows(lgh_ctx *ctx, const lgh_q8 *w, const float *x, const float *nw, float eps, float *y,
                    size_t tokens) {
   const size_t k = w->k, pq = (w->bpr + 3) / 4;
-  // Passes of up to 64 tokens, evenly filled in whole 16-token tiles.
-  const size_t passes = (tokens + 63) / 64, mt = ((tokens + passes - 1) / passes + 15) / 16, chunk = mt * 16;
-  Carve cv;
-  const size_t o_ci = cv.take(mt * pq * 2 * 1024), o_si = cv.take(mt * pq * 256);
-  const bool wanted = lgh::q8_batch_wanted(w, tokens), captured = wanted && capturing(ctx);
-  if (wanted && (cv.off <= ctx->ws_bytes || !captured)) {
-    char *ws = nullptr;
-    if (int r = grow_ws(ctx).get(cv.off, &ws)) return r;
-    ctx->ws_captured = ctx->ws_captured || captured;
-    auto *ci = reinterpret_cast<uint8_t *>(ws + o_ci);
-    auto *si = reinterpret_cast<float *>(ws + o_si);
-    lgh::ActPrologue pro;
-    pro.nw = nw;
-    pro.eps = eps;
-    for (size_t t0 = 0; t0 < tokens; t0 += chunk) {
-      const size_t mc = std::min(chunk, tokens - t0);
-      LGH_HIP(ctx, lgh::launch_act_quant_mma(x + t0 * k, pro, mc, k, 0, ci, si, nullptr, ctx->stream,
-                                             lgh::MmaOrder::kPair));
-      LGH_HIP(ctx, lgh::launch_q8_mma(w, ci, si, y + t0 * w->n, mc, ctx->stream));
-    }
-    return LGH_OK;
-  }
-  if (nw && k > lgh::kQ8GemvMaxK) {  // rows longer than the prologue covers: rms_norm first
+  // Rows longer than the GEMV's norm prologue covers are normed into ctx->ffn
+  // there; sized on either route, so that a captured call that takes the GEMV
+  // finds it as after a GEMV.
+  const bool norm_first = nw && k > lgh::kQ8GemvMaxK;
+  if (norm_first)
     if (int r = ensure(ctx, &ctx->ffn, &ctx->ffn_bytes, tokens * k * sizeof(float))) return r;
+  if (lgh::q8_batch_wanted(w, tokens)) {
+    // Passes of up to 64 tokens, evenly filled in whole 16-token tiles.
+    const size_t passes = (tokens + 63) / 64, mt = ((tokens + passes - 1) / passes + 15) / 16, chunk = mt * 16;
+    const size_t rec = pq * (2 * 1024 + 256);  // codes and scales of a 16-token tile
+    if (char *img = q8_image(ctx, w, mt * rec, 4 * rec)) {
+      auto *ci = reinterpret_cast<uint8_t *>(img);
+      auto *si = reinterpret_cast<float *>(img + mt * pq * 2 * 1024);
+      lgh::ActPrologue pro;
+      pro.nw = nw;
+      pro.eps = eps;
+      for (size_t t0 = 0; t0 < tokens; t0 += chunk) {
+        const size_t mc = std::min(chunk, tokens - t0);
+        LGH_HIP(ctx, lgh::launch_act_quant_mma(x + t0 * k, pro, mc, k, 0, ci, si, nullptr, ctx->stream,
+                                               lgh::MmaOrder::kPair));
+        LGH_HIP(ctx, lgh::launch_q8_mma(w, ci, si, y + t0 * w->n, mc, ctx->stream));
+      }
+      return LGH_OK;
+    }
+  }
+  if (norm_first) {
     float *nd = static_cast<float *>(ctx->ffn);
     LGH_HIP(ctx, lgh::launch_rms_norm(x, nw, k, tokens, eps, nd, ctx->stream));
     x = nd;

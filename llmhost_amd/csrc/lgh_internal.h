@@ -36,7 +36,6 @@
 #include <cstdint>
 #include <mutex>
 #include <string>
-#include <vector>
 
 #include "../../include/llm_gpu_hip.h"
 
@@ -50,10 +49,9 @@ struct lgh_ctx {
   // GEMM workspace: activation operand image, f32 row scales [m], split-K partials.
   void *ws = nullptr;
   size_t ws_bytes = 0;
-  // A captured Q8_0 call holds the workspace's address: growing or trimming it
-  // then keeps the old buffer in `kept`, until the context goes.
-  bool ws_captured = false;
-  std::vector<void *> kept;
+  // Activation image of eager Q8_0 calls of several tokens.
+  void *q8_img = nullptr;
+  size_t q8_img_bytes = 0;
   // Device staging for the host-pointer entry points.
   void *stage = nullptr;
   size_t stage_bytes = 0;
@@ -80,6 +78,14 @@ struct lgh_q8 {
   size_t n = 0, k = 0, bpr = 0;
   int8_t *qs = nullptr;    // n*bpr*32 bytes
   uint16_t *sc = nullptr;
+  // Activation images of captured calls, one each, held as long as the matrix.
+  struct Image {
+    void *p = nullptr;
+    Image *next = nullptr;
+  };
+  Image *images = nullptr;
+  size_t images_bytes = 0;
+  std::mutex images_mu;  // guards both
 };
 
 // ---- internal launchers (return hipError_t of the launch) ----------------

@@ -49,7 +49,7 @@ def test_q8_batch_keeps_tokens_apart(gpu_ctx):
 
 
 def test_q8_batch_under_capture_without_a_workspace(oracle):
-    """A captured call whose image workspace would have to grow takes the GEMV instead."""
+    """A call captured without an eager one before it runs the same pass as an eager one, bit for bit."""
     import torch
 
     n, k, tokens = 8192, 2048, 16
@@ -72,13 +72,17 @@ def test_q8_batch_under_capture_without_a_workspace(oracle):
         graph.replay()
         torch.cuda.synchronize()
         assert_close(y.cpu().numpy(), ref, what="captured q8")
+    got = y.clone()
+    q4.q8_apply(w, x, tokens, y)
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int32), got.view(torch.int32))
     del graph
     w.free()
     ctx.close()
 
 
 def test_q8_batch_graph_survives_growth_and_trim(oracle):
-    """A captured pass keeps its workspace when a later call grows it and when it is trimmed."""
+    """A captured pass keeps its image when later calls grow the context's workspaces and when they are trimmed."""
     import torch
 
     n, k, tokens = 8192, 2048, 16
@@ -116,4 +120,155 @@ def test_q8_batch_graph_survives_growth_and_trim(oracle):
     del graph
     w.free()
     w4.free()
+    ctx.close()
+
+
+def _captured(stream, call):
+    import torch
+
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        call()
+    return graph
+
+
+def test_q4_graph_survives_a_larger_q8_call():
+    """An eager Q8_0 pass whose image is larger than the workspace of a captured Q4 call leaves that
+    workspace alone: what it would have freed is written over before the replay."""
+    import torch
+
+    ctx = q4.Context(0)
+    stream = torch.cuda.Stream()
+    ctx.set_stream(stream.cuda_stream)
+    w4 = q4.Q4Matrix.from_blocks(96, 2048, synth.q4_blocks(6, 96, 2048), ctx)
+    w8 = q4.Q8Matrix.from_blocks(8192, 2048, synth.q8_blocks(5, 8192, 2048), ctx)
+    x4, x8 = (torch.from_numpy(synth.activations(m, m, 2048)).cuda() for m in (8, 64))
+    y4, y8 = torch.zeros(8, 96, device="cuda"), torch.zeros(64, 8192, device="cuda")
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        q4.gemm_q4(w4, x4, y4, 8)
+        torch.cuda.synchronize()
+        ref = y4.clone()
+        graph = _captured(stream, lambda: q4.gemm_q4(w4, x4, y4, 8))
+        for tokens in (32, 64, 33):
+            q4.q8_apply(w8, x8[:tokens].contiguous(), tokens, y8[:tokens])
+            junk = torch.full((1 << 22,), float("nan"), device="cuda")
+            y4.zero_()
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y4.view(torch.int32), ref.view(torch.int32))
+            del junk
+    del graph
+    w4.free()
+    w8.free()
+    ctx.close()
+
+
+def test_q8_graphs_need_the_matrix_only():
+    """Graphs of Q8_0 passes replayed on streams of their own, beside each other and eager calls of
+    their context, and after the context is closed."""
+    import torch
+
+    n, k = 8200, 2080
+    ctx = q4.Context(0)
+    stream = torch.cuda.Stream()
+    ctx.set_stream(stream.cuda_stream)
+    w = q4.Q8Matrix.from_blocks(n, k, synth.q8_blocks(5, n, k), ctx)
+    sizes = (16, 33, 64)
+    xs = [torch.from_numpy(synth.activations(m, m, k)).cuda() for m in sizes]
+    ys = [torch.zeros(m, n, device="cuda") for m in sizes]
+    refs = [torch.zeros(m, n, device="cuda") for m in sizes]
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        for x, r, m in zip(xs, refs, sizes):
+            q4.q8_apply(w, x, m, r)
+        torch.cuda.synchronize()
+        graphs = [_captured(stream, lambda: q4.q8_apply(w, x, m, y)) for x, y, m in zip(xs[:2], ys, sizes)]
+    side = [torch.cuda.Stream() for _ in graphs]
+    for closed in (False, True):
+        for _ in range(4):
+            for y in ys:
+                y.zero_()
+            torch.cuda.synchronize()
+            for _ in range(5):
+                for g, s in zip(graphs, side):
+                    with torch.cuda.stream(s):
+                        g.replay()
+                if not closed:
+                    with torch.cuda.stream(stream):
+                        q4.q8_apply(w, xs[2], 64, ys[2])
+            torch.cuda.synchronize()
+            for y, r in list(zip(ys, refs))[:2 if closed else 3]:
+                assert torch.equal(y.view(torch.int32), r.view(torch.int32))
+        if not closed:
+            ctx.close()
+    del graphs
+    w.free()
+
+
+def test_q8_capture_and_trim_give_the_workspace_back():
+    """A captured pass holds its image, not the context's workspaces: trimming returns those, however
+    often a pass is captured."""
+    import torch
+
+    n, k = 8192, 2048
+    ctx = q4.Context(0)
+    stream = torch.cuda.Stream()
+    ctx.set_stream(stream.cuda_stream)
+    w = q4.Q8Matrix.from_blocks(n, k, synth.q8_blocks(5, n, k), ctx)
+    w4 = q4.Q4Matrix.from_blocks(64, 4096, synth.q4_blocks(6, 64, 4096), ctx)
+    w4.prepare_gemm()
+    m = 16384  # an activation image of over 100 MB
+    x, y = torch.zeros(16, k, device="cuda"), torch.zeros(16, n, device="cuda")
+    x4, y4 = torch.zeros(m, 4096, device="cuda"), torch.zeros(m, 64, device="cuda")
+    torch.cuda.synchronize()
+    graphs, free = [], []
+    with torch.cuda.stream(stream):
+        for _ in range(8):
+            q4.gemm_q4(w4, x4, y4, m)
+            q4.q8_apply(w, x, 16, y)
+            torch.cuda.synchronize()
+            graphs.append(_captured(stream, lambda: q4.q8_apply(w, x, 16, y)))
+            ctx.trim()
+            free.append(torch.cuda.mem_get_info()[0])
+    assert free[0] - free[-1] < 100 << 20
+    del graphs
+    w.free()
+    w4.free()
+    ctx.close()
+
+
+def test_q8_captured_images_are_bounded():
+    """Past the bytes a matrix holds for captured calls a call takes the GEMV: rows as of one token."""
+    import torch
+
+    n, k, tokens, calls = 8192, 16384, 64, 60  # 1.1 MiB an image: 56 or 57 fit in 64 MiB
+    ctx = q4.Context(0)
+    stream = torch.cuda.Stream()
+    ctx.set_stream(stream.cuda_stream)
+    w = q4.Q8Matrix.from_blocks(n, k, synth.q8_blocks(5, n, k), ctx)
+    x = torch.from_numpy(synth.activations(3, tokens, k)).cuda()
+    ys = torch.zeros(calls, tokens, n, device="cuda")
+    many, one = torch.zeros(tokens, n, device="cuda"), torch.zeros(tokens, n, device="cuda")
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        def step():
+            for y in ys:
+                q4.q8_apply(w, x, tokens, y)
+
+        graph = _captured(stream, step)
+        q4.q8_apply(w, x, tokens, many)
+        for t in range(tokens):
+            q4.q8_apply(w, x[t], 1, one[t])
+        for _ in range(2):
+            ys.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            for i in (0, 1, 40, 55):
+                assert torch.equal(ys[i].view(torch.int32), many.view(torch.int32))
+            for i in (58, 59):
+                assert torch.equal(ys[i].view(torch.int32), one.view(torch.int32))
+    del graph
+    w.free()
     ctx.close()

@@ -757,6 +757,20 @@ struct ActIn {
   float *tmp = nullptr;
 };
 
+// Whether an output of the call shares memory with the rows x or the norm weight
+// nw: a kernel that norms x in every workgroup would read what others have
+// already written, so such calls norm into a copy first.
+static bool norms_in_place(const lgh_q4 *const *w, int nmat, const float *x, const float *nw, float *const *y,
+                           size_t m) {
+  auto meet = [](const float *a, size_t na, const float *b, size_t nb) {
+    const auto pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
+    return na && nb && pa < pb + nb * sizeof(float) && pb < pa + na * sizeof(float);
+  };
+  for (int j = 0; nw && j < nmat; j++)
+    if (meet(y[j], m * w[j]->n, x, m * w[j]->k) || meet(y[j], m * w[j]->n, nw, w[j]->k)) return true;
+  return false;
+}
+
 static int gemm_multi_dev(lgh_ctx *ctx, const Ws &wsp, const lgh_q4 *const *w, int nmat, ActIn in,
                           float *const *y_dev, size_t m, int mode);
 static int mma_chunked(lgh_ctx *ctx, const Ws &wsp, const lgh_q4 *const *w, int nmat, const float *x_dev,
@@ -988,7 +1002,8 @@ static int gemm_multi_dev(lgh_ctx *ctx, const Ws &wsp, const lgh_q4 *const *w, i
   if (int r = set_device(ctx)) return r;
   // Small batches are weight-stream bound: nibble planes, no operand image.
   if (lgh::plan_q4_batch(m, bpr).ok) {  // m <= 4: dot4 on the nibble planes
-    if (!in.u && lgh::q4_batch_norms(bpr)) {  // the rows normed and quantized inside the kernel
+    if (!in.u && lgh::q4_batch_norms(bpr) && !norms_in_place(w, nmat, in.x, in.nw, y_dev, m)) {
+      // The rows normed and quantized inside the kernel.
       LGH_HIP(ctx, lgh::launch_q4_gemv_batch(w, y_dev, nmat, in.x, nullptr, nullptr, in.nw, in.eps, m, mode,
                                              ctx->act_mode, ctx->stream));
       return LGH_OK;
@@ -1656,7 +1671,7 @@ int lgh_q4_norm_gemv_dev(lgh_ctx *ctx, size_t nmat, const lgh_q4 *const *w, cons
   // One token whose rows fit one K slice: a single launch (norm in the
   // prologue, one act-quant shared by every matrix).
   if (tokens == 1 && k > 0 && w[0]->bpr <= lgh::kFfnMaxBpr && lgh::plan_q4_gemv(rows, w[0]->bpr, 1).ok &&
-      !lgh::q4_gemv_quantize_once(rows, w[0]->bpr, 1)) {
+      !lgh::q4_gemv_quantize_once(rows, w[0]->bpr, 1) && !norms_in_place(w, nm, hidden_dev, norm_w_dev, y_dev, 1)) {
     LGH_HIP(ctx, lgh::launch_q4_gemv_multi(w, y_dev, nm, hidden_dev, nullptr, nullptr, norm_w_dev, eps, mode,
                                            ctx->act_mode, ctx->stream));
     return LGH_OK;

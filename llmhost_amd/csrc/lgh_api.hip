@@ -757,18 +757,29 @@ struct ActIn {
   float *tmp = nullptr;
 };
 
+// Whether na floats at a and nb floats at b share memory.
+static bool share_memory(const float *a, size_t na, const float *b, size_t nb) {
+  const auto pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
+  return na && nb && pa < pb + nb * sizeof(float) && pb < pa + na * sizeof(float);
+}
+
 // Whether an output of the call shares memory with the rows x or the norm weight
 // nw: a kernel that norms x in every workgroup would read what others have
 // already written, so such calls norm into a copy first.
 static bool norms_in_place(const lgh_q4 *const *w, int nmat, const float *x, const float *nw, float *const *y,
                            size_t m) {
-  auto meet = [](const float *a, size_t na, const float *b, size_t nb) {
-    const auto pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
-    return na && nb && pa < pb + nb * sizeof(float) && pb < pa + na * sizeof(float);
-  };
   for (int j = 0; nw && j < nmat; j++)
-    if (meet(y[j], m * w[j]->n, x, m * w[j]->k) || meet(y[j], m * w[j]->n, nw, w[j]->k)) return true;
+    if (share_memory(y[j], m * w[j]->n, x, m * w[j]->k) || share_memory(y[j], m * w[j]->n, nw, w[j]->k)) return true;
   return false;
+}
+
+// Matrices a launch: all of the call's, or one after another, as the reference's
+// calls, where two outputs share memory (each adding to the same rows, say).
+static int launch_group(const lgh_q4 *const *w, int nmat, float *const *y, size_t m) {
+  for (int i = 0; i < nmat; i++)
+    for (int j = 0; j < i; j++)
+      if (share_memory(y[i], m * w[i]->n, y[j], m * w[j]->n)) return 1;
+  return nmat;
 }
 
 static int gemm_multi_dev(lgh_ctx *ctx, const Ws &wsp, const lgh_q4 *const *w, int nmat, ActIn in,
@@ -935,6 +946,7 @@ static int mma_chunked(lgh_ctx *ctx, const Ws &wsp, const lgh_q4 *const *w, int 
   // the f32 summation order.  A fixed scratch too small for the chunk's image
   // fails in wsp.get.
   const size_t chunk = std::min<size_t>(m, 64);
+  const int group = launch_group(w, nmat, y_dev, m);
   const Layout lay = layout(chunk);
   char *ws = nullptr;
   if (int r = wsp.get(lay.bytes, &ws)) return r;
@@ -949,7 +961,8 @@ static int mma_chunked(lgh_ctx *ctx, const Ws &wsp, const lgh_q4 *const *w, int 
                                              reinterpret_cast<float *>(ws + lay.o_rs), ctx->stream));
     float *yc[3] = {nullptr, nullptr, nullptr};
     for (int j = 0; j < nmat; j++) yc[j] = w[j]->n ? y_dev[j] + m0 * w[j]->n : nullptr;
-    LGH_HIP(ctx, lgh::launch_q4_gemv_mma(w, yc, nmat, ci, si, mc, mode, ctx->stream, true));
+    for (int j = 0; j < nmat; j += group)
+      LGH_HIP(ctx, lgh::launch_q4_gemv_mma(w + j, yc + j, group, ci, si, mc, mode, ctx->stream, true));
   }
   return LGH_OK;
 }
@@ -1001,11 +1014,18 @@ static int gemm_multi_dev(lgh_ctx *ctx, const Ws &wsp, const lgh_q4 *const *w, i
   }
   if (int r = set_device(ctx)) return r;
   // Small batches are weight-stream bound: nibble planes, no operand image.
+  const int group = launch_group(w, nmat, y_dev, m);
   if (lgh::plan_q4_batch(m, bpr).ok) {  // m <= 4: dot4 on the nibble planes
+    auto batch = [&](const float *x, const int8_t *qs, const float *sc, const float *nw, int per_row) {
+      for (int j = 0; j < nmat; j += group)
+        if (hipError_t e = lgh::launch_q4_gemv_batch(w + j, y_dev + j, group, x, qs, sc, nw, in.eps, m, mode, per_row,
+                                                     ctx->stream))
+          return e;
+      return hipSuccess;
+    };
     if (!in.u && lgh::q4_batch_norms(bpr) && !norms_in_place(w, nmat, in.x, in.nw, y_dev, m)) {
       // The rows normed and quantized inside the kernel.
-      LGH_HIP(ctx, lgh::launch_q4_gemv_batch(w, y_dev, nmat, in.x, nullptr, nullptr, in.nw, in.eps, m, mode,
-                                             ctx->act_mode, ctx->stream));
+      LGH_HIP(ctx, batch(in.x, nullptr, nullptr, in.nw, ctx->act_mode));
       return LGH_OK;
     }
     if (int r = materialize(ctx, in, m, k, &x_dev)) return r;
@@ -1018,12 +1038,10 @@ static int gemm_multi_dev(lgh_ctx *ctx, const Ws &wsp, const lgh_q4 *const *w, i
       auto *sc = reinterpret_cast<float *>(ws + os);
       LGH_HIP(ctx, lgh::launch_act_quant(x_dev, m, k, ctx->act_mode, qs, sc, nullptr,
                                          reinterpret_cast<float *>(ws + orow), ctx->stream));
-      LGH_HIP(ctx, lgh::launch_q4_gemv_batch(w, y_dev, nmat, nullptr, qs, sc, nullptr, 0.0f, m, mode, 0,
-                                             ctx->stream));
+      LGH_HIP(ctx, batch(nullptr, qs, sc, nullptr, 0));
       return LGH_OK;
     }
-    LGH_HIP(ctx, lgh::launch_q4_gemv_batch(w, y_dev, nmat, x_dev, nullptr, nullptr, nullptr, 0.0f, m, mode,
-                                           ctx->act_mode, ctx->stream));
+    LGH_HIP(ctx, batch(x_dev, nullptr, nullptr, nullptr, ctx->act_mode));
     return LGH_OK;
   }
   if (lgh::plan_q4_mma(nmax, m, bpr).ok) {  // m <= 64: activation image, then int8 MFMA per block
@@ -1037,7 +1055,8 @@ static int gemm_multi_dev(lgh_ctx *ctx, const Ws &wsp, const lgh_q4 *const *w, i
     auto *si = reinterpret_cast<float *>(ws + o_si);
     LGH_HIP(ctx, lgh::launch_act_quant_mma(x_dev, pro, m, k, ctx->act_mode, ci, si,
                                            reinterpret_cast<float *>(ws + o_rs), ctx->stream));
-    LGH_HIP(ctx, lgh::launch_q4_gemv_mma(w, y_dev, nmat, ci, si, m, mode, ctx->stream));
+    for (int j = 0; j < nmat; j += group)
+      LGH_HIP(ctx, lgh::launch_q4_gemv_mma(w + j, y_dev + j, group, ci, si, m, mode, ctx->stream));
     return LGH_OK;
   }
   for (int j = 0; j < nmat; j++)

@@ -1241,12 +1241,6 @@ static char *q8_image(lgh_ctx *ctx, const lgh_q8 *wc, size_t bytes, size_t full)
 static int q8_rows(lgh_ctx *ctx, const lgh_q8 *w, const float *x, const float *nw, float eps, float *y,
                    size_t tokens) {
   const size_t k = w->k, pq = (w->bpr + 3) / 4;
-  // Rows longer than the GEMV's norm prologue covers are normed into ctx->ffn
-  // there; sized on either route, so that a captured call that takes the GEMV
-  // finds it as after a GEMV.
-  const bool norm_first = nw && k > lgh::kQ8GemvMaxK;
-  if (norm_first)
-    if (int r = ensure(ctx, &ctx->ffn, &ctx->ffn_bytes, tokens * k * sizeof(float))) return r;
   if (lgh::q8_batch_wanted(w, tokens)) {
     // Passes of up to 64 tokens, evenly filled in whole 16-token tiles.
     const size_t passes = (tokens + 63) / 64, mt = ((tokens + passes - 1) / passes + 15) / 16, chunk = mt * 16;
@@ -1266,7 +1260,8 @@ static int q8_rows(lgh_ctx *ctx, const lgh_q8 *w, const float *x, const float *n
       return LGH_OK;
     }
   }
-  if (norm_first) {
+  if (nw && k > lgh::kQ8GemvMaxK) {  // rows longer than the prologue covers: rms_norm first
+    if (int r = ensure(ctx, &ctx->ffn, &ctx->ffn_bytes, tokens * k * sizeof(float))) return r;
     float *nd = static_cast<float *>(ctx->ffn);
     LGH_HIP(ctx, lgh::launch_rms_norm(x, nw, k, tokens, eps, nd, ctx->stream));
     x = nd;

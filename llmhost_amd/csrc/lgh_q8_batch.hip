@@ -13,9 +13,11 @@
 //     would take, and every result is one exact block dot;
 //   * the terms (f32(dot) * sw) * sa are added in block order within a quad of
 //     blocks (weights.rs:206-212), the last product fused into the addition, two
-//     quads to a chunk, and the chunks' sums in two sums in turn: as close to the
-//     64-bit result as the GEMV's 16 partial sums (one running sum over the row
-//     was 1.7 times as far from it).
+//     quads to a chunk, and the chunks' sums in two sums in turn; rows of more than
+//     80 blocks are summed so in groups of 64 blocks.  Relative error (2-norms)
+//     against 64 bits, here and of the GEMV's partial sums: K=1536 7.0e-8, 6.9e-8;
+//     K=4128 8.1e-8, 8.4e-8; K=8192 8.3e-8, 8.6e-8; K=16384 9.2e-8, 9.4e-8
+//     (without the groups 8.4e-8, 9.8e-8 and 1.2e-7 at the last three).
 // A wave owns 16 rows and walks them chunk by chunk (4.3 KB of weights); the 8
 // waves of a workgroup share the activations, staged in LDS KS blocks at a
 // time.  HBM-bound: norm + head, K=1536, N=65536 (107 MB), M = 2 / 16 / 32 / 64:
@@ -43,7 +45,9 @@ struct Q8MmaArgs {
   int vec4;            // n % 4 == 0 and y 16-byte aligned
 };
 
-constexpr int kChunk = 8;  // blocks of a chunk
+constexpr int kChunk = 8;   // blocks of a chunk
+constexpr int kGroup = 64;  // blocks of a group of chunks
+constexpr int kLong = 80;   // rows of more blocks are summed by groups
 
 // Weights of one chunk of 16 rows: four block pairs, two block scales.
 struct Q8Chunk {
@@ -70,8 +74,9 @@ __device__ __forceinline__ void q8_load(__amdgpu_buffer_rsrc_t wr, __amdgpu_buff
   }
 }
 
-// TT 16-token tiles, W waves, KS blocks of activations in LDS.
-template <int TT, int W, int KS>
+// TT 16-token tiles, W waves, KS blocks of activations in LDS.  LONG: rows of
+// more than kLong blocks, whose chunks are summed group by group.
+template <int TT, int W, int KS, bool LONG>
 __global__ __launch_bounds__(W * kWave) __attribute__((amdgpu_waves_per_eu(4))) void q8_mma_kernel(Q8MmaArgs a) {
   static_assert(KS % kChunk == 0, "whole chunks per stage");
   constexpr int THREADS = W * kWave;
@@ -91,10 +96,24 @@ __global__ __launch_bounds__(W * kWave) __attribute__((amdgpu_waves_per_eu(4))) 
   const auto ar = make_rsrc(a.si, static_cast<uint32_t>(a.mt * a.pq) * 256u);
 
   float acc[2][TT][4];  // sums of every other chunk, in turns
+  // LONG: the sums of the groups before; of four token tiles in LDS, where the
+  // registers are used up and two workgroups a CU still fit.
+  constexpr bool kTotLds = LONG && TT == 4;
+  __shared__ float s_tot[kTotLds ? TT * 4 : 1][kTotLds ? THREADS : 1];
+  float r_tot[LONG && !kTotLds ? TT : 1][4];
+  auto tot = [&](int tt, int v) -> float & {
+    if constexpr (kTotLds)
+      return s_tot[tt * 4 + v][tid];
+    else
+      return r_tot[tt][v];
+  };
 #pragma unroll
   for (int tt = 0; tt < TT; tt++)
 #pragma unroll
-    for (int v = 0; v < 4; v++) acc[0][tt][v] = acc[1][tt][v] = 0.0f;
+    for (int v = 0; v < 4; v++) {
+      acc[0][tt][v] = acc[1][tt][v] = 0.0f;
+      if constexpr (LONG) tot(tt, v) = 0.0f;
+    }
 
   // A stage's activations, every load of a tile before its first LDS write.
   // Pairs and quads past the row's image hold 0: whole chunks are computed, and
@@ -174,6 +193,17 @@ __global__ __launch_bounds__(W * kWave) __attribute__((amdgpu_waves_per_eu(4))) 
           acc[1][tt][v] = acc[0][tt][v];
           acc[0][tt][v] = t;
         }
+      if constexpr (LONG) {
+        if ((s0 + kc) % kGroup == kGroup - kChunk) {  // uniform: a group is done
+#pragma unroll
+          for (int tt = 0; tt < TT; tt++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+              tot(tt, v) += acc[0][tt][v] + acc[1][tt][v];
+              acc[0][tt][v] = acc[1][tt][v] = 0.0f;
+            }
+        }
+      }
       q8_load(wr, sr, bpr, s0 + kc + kChunk, c);
     }
     s0 += KS;
@@ -191,7 +221,10 @@ __global__ __launch_bounds__(W * kWave) __attribute__((amdgpu_waves_per_eu(4))) 
     float *y = a.y + static_cast<size_t>(t) * a.n + row0 + 4 * g;
     float o[4];
 #pragma unroll
-    for (int v = 0; v < 4; v++) o[v] = acc[0][tt][v] + acc[1][tt][v];
+    for (int v = 0; v < 4; v++) {
+      o[v] = acc[0][tt][v] + acc[1][tt][v];
+      if constexpr (LONG) o[v] += tot(tt, v);
+    }
     if (a.vec4 && 4 * g + 3 < rows) {
       *reinterpret_cast<float4 *>(y) = make_float4(o[0], o[1], o[2], o[3]);
     } else {
@@ -206,7 +239,10 @@ template <int TT, int KS>
 hipError_t launch_tt(const Q8MmaArgs &a, hipStream_t st) {
   constexpr int W = 8;
   const unsigned wgs = static_cast<unsigned>((a.n + 16 * W - 1) / (16 * W));
-  hipLaunchKernelGGL((q8_mma_kernel<TT, W, KS>), dim3(wgs), dim3(W * kWave), 0, st, a);
+  if (a.bpr > kLong)
+    hipLaunchKernelGGL((q8_mma_kernel<TT, W, KS, true>), dim3(wgs), dim3(W * kWave), 0, st, a);
+  else
+    hipLaunchKernelGGL((q8_mma_kernel<TT, W, KS, false>), dim3(wgs), dim3(W * kWave), 0, st, a);
   return hipGetLastError();
 }
 
@@ -218,12 +254,13 @@ hipError_t launch_tt(const Q8MmaArgs &a, hipStream_t st) {
 // saves have to be worth the chain: measured crossings at K=1024, N=32003
 // (35 MB) between 2 and 3 tokens (13.4 against 13.0 us, 18.7 against 13), at
 // K=1536, N=65536 below 2 (30.9 against 24.0 us), at K=2048, N=8192 (18 MB) at 5
-// (16 against 14 us at 6).  Fewer rows leave most CUs without a workgroup.
+// (16 against 14 us at 6).  Fewer rows leave most CUs without a workgroup.  Rows
+// longer than one launch of the GEMV covers stay with its K ranges, whose sums
+// are closer to the 64-bit result there.
 bool q8_batch_wanted(const lgh_q8 *w, size_t tokens) {
   const size_t chunks = (w->bpr + kChunk - 1) / kChunk;
-  return tokens >= 2 && w->bpr > 0 && w->n >= 8192 &&
-         (tokens - 1) * (w->n * w->bpr * 34) >= ((size_t{32} + 8 * chunks) << 20) &&
-         w->bpr < (size_t{1} << 20);  // a 64-token image stays below 2^31 bytes
+  return tokens >= 2 && w->bpr > 0 && w->k <= kQ8GemvMaxK && w->n >= 8192 &&
+         (tokens - 1) * (w->n * w->bpr * 34) >= ((size_t{32} + 8 * chunks) << 20);
 }
 
 hipError_t launch_q8_mma(const lgh_q8 *w, const uint8_t *codes, const float *scales, float *y, size_t m,

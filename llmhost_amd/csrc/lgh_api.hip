@@ -1210,10 +1210,11 @@ constexpr size_t kQ8CapturedBytes = size_t(64) << 20;
 // replayed on any stream, beside other calls and graphs, and after the context
 // is gone.  It belongs to the matrix, without which the graph is not good either.
 static char *q8_image(lgh_ctx *ctx, const lgh_q8 *wc, size_t bytes, size_t full) {
+  const bool captured = capturing(ctx);
+  if (!captured && full <= ctx->q8_img_bytes) return static_cast<char *>(ctx->q8_img);
   AllocUnderCapture relaxed;
-  if (!capturing(ctx)) {
-    if (full <= ctx->q8_img_bytes || ensure(ctx, &ctx->q8_img, &ctx->q8_img_bytes, full) == LGH_OK)
-      return static_cast<char *>(ctx->q8_img);
+  if (!captured) {
+    if (ensure(ctx, &ctx->q8_img, &ctx->q8_img_bytes, full) == LGH_OK) return static_cast<char *>(ctx->q8_img);
     (void)hipGetLastError();
     return nullptr;
   }

@@ -1473,10 +1473,20 @@ static int ffn_fused(lgh_ctx *ctx, const lgh_q4 *w1, const lgh_q4 *w3, const lgh
   const bool codes = ctx->act_mode == LGH_ACT_PER_BLOCK &&
                      (m == 1 ? lgh::plan_q4_gemv(w2->n, w2->bpr, 1).ok
                              : lgh::plan_q4_batch(m, w2->bpr).ok && lgh::q4_batch_quantize_once(w2->bpr));
+  // For several tokens what the f32 form needs is sized with codes too (unused
+  // then): a shape that ran once needs no growth in either act-quant mode.
   Carve cv;
   const size_t o_q = cv.take(m * n), o_s = cv.take(m * (n / 32) * sizeof(float));
-  const size_t o_f = cv.take(codes ? 0 : m * n * sizeof(float));
+  const size_t o_f = cv.take(codes && m == 1 ? 0 : m * n * sizeof(float));
   if (int r = ensure(ctx, &ctx->ffn, &ctx->ffn_bytes, cv.off)) return r;
+  if (codes && m > 1) {
+    Carve wv;  // the down projection's codes, as gemm_multi_dev lays them out
+    wv.take(m * n);
+    wv.take(m * w2->bpr * sizeof(float));
+    wv.take(m * sizeof(float));
+    char *ws = nullptr;
+    if (int r = grow_ws(ctx).get(wv.off, &ws)) return r;
+  }
   char *f = static_cast<char *>(ctx->ffn);
   auto *hq = reinterpret_cast<int8_t *>(f + o_q);
   auto *hs = reinterpret_cast<float *>(f + o_s);

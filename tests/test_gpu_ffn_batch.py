@@ -43,3 +43,47 @@ def test_ffn_few_tokens_equals_op_sequence(gpu_ctx, dim, inter, tokens, norm, pe
         for w in (w1, w3, w2):
             w.free()
     assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("warm,captured", [("PerBlock", "PerRow"), ("PerRow", "PerBlock")])
+@pytest.mark.parametrize("dim,inter,tokens", [(1536, 8192, 2), (96, 2080, 4), (96, 10752, 3),
+                                              (544, 2048, 4), (1056, 2272, 9), (64, 8224, 385)])
+def test_ffn_shape_that_ran_once_is_captured_in_either_mode(dim, inter, tokens, warm, captured):
+    """A block run eagerly in one act-quant mode needs no workspace to grow in the other: its capture
+    is accepted and its replays equal an eager call."""
+    import torch
+
+    ctx = q4.Context(0)
+    stream = torch.cuda.Stream()
+    ctx.set_stream(stream.cuda_stream)
+    w1, w3, w2 = (q4.Q4Matrix.from_blocks(n, k, synth.q4_blocks(n + i, n, k), ctx)
+                  for i, (n, k) in enumerate(((inter, dim), (inter, dim), (dim, inter))))
+    x = torch.from_numpy(synth.activations(60 + tokens, tokens, dim)).cuda()
+    hidden = x.clone()
+    torch.cuda.synchronize()
+
+    def block():
+        q4.ffn_residual(w1, w3, w2, None, 1e-5, hidden, tokens)
+
+    with torch.cuda.stream(stream):
+        q4.set_act_quant(q4.ActQuant[warm], ctx)
+        block()
+        q4.set_act_quant(q4.ActQuant[captured], ctx)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            block()
+        got = []
+        for _ in range(3):
+            hidden.copy_(x)
+            graph.replay()
+            got.append(hidden.clone())
+        hidden.copy_(x)
+        block()
+        torch.cuda.synchronize()
+        for g in got:
+            assert torch.equal(g.view(torch.int32), hidden.view(torch.int32))
+    del graph
+    for w in (w1, w3, w2):
+        w.free()
+    ctx.close()

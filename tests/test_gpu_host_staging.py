@@ -17,12 +17,11 @@ def test_host_call_equals_device_call(gpu_ctx, m, n, k, add):
     import torch
 
     w = q4.Q4Matrix.from_blocks(n, k, synth.q4_blocks(n + k, n, k), gpu_ctx)
-    x = synth.activations(m, m, k)
-    y = synth.activations(m + 1, m, n)
     call = q4.gemm_q4_add if add else q4.gemm_q4
-    dx, dy = torch.from_numpy(x).cuda(), torch.from_numpy(y).cuda()
-    for _ in range(2):  # the staging buffer is used again
-        hy, dz = y.copy(), dy.clone()
+    for i in range(3):  # the staging buffer is used again, for other values
+        x = synth.activations(m + 10 * i, m, k)
+        hy = synth.activations(m + 10 * i + 1, m, n)
+        dx, dz = torch.from_numpy(x).cuda(), torch.from_numpy(hy).cuda()
         call(w, x, hy, m)
         call(w, dx, dz, m)
         torch.cuda.synchronize()

@@ -2,7 +2,8 @@
 bit: every token slot count, rows that end inside a block group, a down projection whose kernel
 takes codes (inter 2080-8192), f32 rows (shorter) or the matrix-core batch route (longer); from 5
 tokens on, one and two token tiles, block counts of h that pad its image's quad by 0 to 3, rows of
-33 to 65 blocks and one more slice chunk; both act-quant modes, with and without the norm."""
+33 to 65 blocks and one more slice chunk, of 192 (the longest that one token tile fuses), 193 and 257;
+both act-quant modes, with and without the norm."""
 
 import numpy as np
 import pytest
@@ -17,7 +18,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("dim,inter,tokens", [(2048, 8192, 2), (1536, 8192, 3), (96, 2080, 4), (544, 2048, 2),
                                               (1056, 64, 4), (2048, 10752, 3), (1536, 8224, 4),
                                               (1536, 8192, 13), (1056, 128, 5), (2048, 160, 16), (2080, 192, 17),
-                                              (1568, 2272, 32), (4128, 256, 9)])
+                                              (1568, 2272, 32), (4128, 256, 9),
+                                              (6144, 160, 9), (6176, 160, 9), (6176, 160, 20), (8224, 128, 32)])
 def test_ffn_few_tokens_equals_op_sequence(gpu_ctx, dim, inter, tokens, norm, per_row):
     shapes = ((inter, dim), (inter, dim), (dim, inter))
     w1, w3, w2 = (q4.Q4Matrix.from_blocks(n, k, synth.q4_blocks(50 + i + n, n, k), gpu_ctx)

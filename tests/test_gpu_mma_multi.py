@@ -1,6 +1,7 @@
 """Several matrices in one matrix-core batch launch (5 to 64 tokens) equal one launch each, bit for
 bit: matrices of one plan, a matrix whose own plan differs (three token tiles past 8192 rows), rows
-that end inside a 16-row tile, every number of token tiles."""
+that end inside a 16-row tile, every number of token tiles, rows long enough for the form that loads
+ahead (one and four token tiles)."""
 
 import numpy as np
 import pytest
@@ -12,7 +13,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("k,rows,tokens", [(2048, (2048, 512, 512), 40), (1568, (33, 1, 100), 5),
                                            (1536, (8200, 256, 8192), 37), (1536, (64, 8208, 8224), 48),
-                                           (4096, (96, 130, 17), 64), (96, (48, 16), 17)])
+                                           (4096, (96, 130, 17), 64), (96, (48, 16), 17),
+                                           (6176, (130, 33, 17), 9), (6176, (130, 33, 17), 53)])
 def test_norm_gemv_equals_one_matrix_at_a_time(gpu_ctx, k, rows, tokens):
     ws = [q4.Q4Matrix.from_blocks(n, k, synth.q4_blocks(70 + i + n, n, k), gpu_ctx) for i, n in enumerate(rows)]
     x = synth.activations(71 + tokens, tokens, k)

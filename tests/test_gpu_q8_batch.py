@@ -33,6 +33,22 @@ def test_q8_batch_matches_oracle(gpu_ctx, oracle, n, k, tokens, norm):
     assert_close(y, ref, what=f"q8 {n}x{k} m={tokens}")
 
 
+def test_q8_batch_random_shapes(gpu_ctx, oracle):
+    """Seeded sizes on both sides of the pass's rule, as the fuzz of the other routes."""
+    rng = np.random.default_rng(20261204)
+    for i in range(12):
+        n, k, tokens = int(rng.integers(8192, 9300)), 32 * int(rng.integers(1, 140)), int(rng.integers(2, 131))
+        print(f"[q8 fuzz {i}] n={n} k={k} tokens={tokens}", flush=True)
+        blocks = synth.q8_blocks(i, n, k)
+        x = synth.activations(100 + i, tokens, k)
+        w = q4.Q8Matrix.from_blocks(n, k, blocks, gpu_ctx)
+        y = np.zeros((tokens, n), dtype=np.float32)
+        q4.q8_apply(w, x, tokens, y)
+        w.free()
+        ref = oracle.q8_apply(blocks, n, k, x, tokens, threads=8).reshape(tokens, n)
+        assert_close(y, ref, what=f"q8 {n}x{k} m={tokens}")
+
+
 @pytest.mark.parametrize("k,tokens", [(2080, 20), (2592, 48), (4128, 33), (8192, 16), (8192, 64), (16384, 40)])
 def test_q8_batch_is_as_exact_as_one_token(gpu_ctx, oracle, k, tokens):
     """Rows of several tokens are no further from the 64-bit sums of the same codes than those of one

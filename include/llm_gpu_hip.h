@@ -338,8 +338,8 @@ int lgh_q4_ffn_residual_dev(lgh_ctx *ctx, const lgh_q4 *w1, const lgh_q4 *w3, co
  * applied by the launch that writes the shared activation image).
  * Results equal that sequence, also where an output of the _dev call is hidden
  * itself (with norm_w; the rows are then normed into a copy first).  Outputs
- * that share memory are written one matrix after another for 2 to 64 tokens;
- * for one token and for more than 64 they must not. */
+ * that share memory are written one matrix after another for 2 to 48 tokens;
+ * for one token and for more than 48 they must not. */
 int lgh_q4_norm_gemv(lgh_ctx *ctx, size_t nmat, const lgh_q4 *const *w, const float *norm_w, float eps,
                      const float *hidden, float *const *y, size_t tokens, int mode);
 int lgh_q4_norm_gemv_dev(lgh_ctx *ctx, size_t nmat, const lgh_q4 *const *w, const float *norm_w_dev, float eps,

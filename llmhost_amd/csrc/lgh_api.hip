@@ -1540,7 +1540,7 @@ static int ffn_mma_glu(lgh_ctx *ctx, const lgh_q4 *w1, const lgh_q4 *w3, const l
 static int ffn_glu(lgh_ctx *ctx, const lgh_q4 *w1, const lgh_q4 *w3, const lgh_q4 *w2, const float *norm_w_dev,
                    float eps, float *hidden_dev, size_t m, uint8_t *img, bool *done) {
   *done = false;
-  const size_t dim = w1->k, inter = w1->n, mt = (m + 31) / 32;
+  const size_t dim = w1->k, mt = (m + 31) / 32;
   const size_t rec_x = w1->pp * lgh::kMxARec, rec_h = w2->pp * lgh::kMxARec;
   auto gemm = [&](const lgh_q4 *w) {  // m takes the GEMM route, in one chunk
     return !lgh::plan_q4_batch(m, w->bpr).ok && !lgh::plan_q4_mma(w->n, m, w->bpr).ok && mx_fits(w) &&
@@ -1570,7 +1570,7 @@ static int ffn_glu(lgh_ctx *ctx, const lgh_q4 *w1, const lgh_q4 *w3, const lgh_q
   LGH_HIP(ctx, lgh::launch_act_quant_mx(hidden_dev, pro, m, dim, 0, mxa, nullptr, ctx->stream));
   LGH_HIP(ctx, lgh::launch_q4_glu(w1, w3, mxa, m, img, ctx->stream));
   LGH_HIP(ctx, lgh::launch_q4_gemm(&w2, 1, img, &hidden_dev, m, LGH_ADD_F64, plan, part, part_floats, ctx->stream));
-  *done = inter > 0;
+  *done = true;
   return LGH_OK;
 }
 

@@ -468,6 +468,8 @@ __global__ __launch_bounds__(kThreads * KG) __attribute__((amdgpu_waves_per_eu(W
 // tile) x 64 tokens.  A stage holds W1's two records, W3's two, each pair
 // padded to 4 KB so that a wave load reads one matrix, then two activation
 // records: 15 wave loads, the 16 KB of the wide launch.
+// The whole block, the two launches and the one: dim 2048, inter 10752, M = 97 / 256
+// / 512 / 768 52.6 / 78.2 / 130.2 / 171.0 -> 51.6 / 71.3 / 118.9 / 157.3 us.
 struct GluCfg {
   static constexpr int WPW = 4;
   static constexpr int W_STRIDE = 4096;
@@ -506,7 +508,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) v
   const int wave = uniform(threadIdx.x >> 6), wn = wave & 1, wm = wave >> 1;
   const int nt0 = blockIdx.x * 2, mt0 = blockIdx.y * 2;
   const int lane = threadIdx.x & 63, tok = lane & 31, half = lane >> 5;
-  s_hl[threadIdx.x] = hl_table_entry(threadIdx.x);
+  s_hl[threadIdx.x] = hl_table_entry(threadIdx.x);  // ordered by the first stage's barrier (pp >= 1)
 
   float acc[2][1][16];
 #pragma unroll
@@ -556,7 +558,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) v
   for (int u = 0; u < NB - 1; u++)
     if (p + u < pend) step(p + u, lds[u], lds[(u + NB - 1) % NB]);
   asm volatile("s_waitcnt vmcnt(0)" : : : "memory");  // as in q4_gemm_mx_kernel
-  if (a.g.pp < 1) __syncthreads();                    // the table, where no stage's barrier ordered it
 
   // Lane: token tok, elements 8 q + 4 half + e of block nt0 + wn.  Tokens past
   // m and rows past n have g = u = 0, h = 0: code 0, scale 0, the image's padding.
@@ -844,8 +845,9 @@ hipError_t launch_q4_gemm(const lgh_q4 *const *w, int nmat, const uint8_t *mxa, 
 
 // Without split K or K groups: those add an element's parts in another f32
 // order, and the block's results stay the general path's bits.  That leaves
-// launches of >= 512 128 x 32 tiles, where it won at every size measured
-// (figures above q4_glu_mx_kernel), down to 256 workgroups.
+// launches of >= 512 128 x 32 tiles of the general path (256 workgroups here),
+// where it won at every size measured (figures above GluCfg), and rows of one
+// block pair (K <= 64), which have no K groups, at any number of tiles.
 bool q4_glu_wanted(const lgh_q4 *w1, const lgh_q4 *w3, size_t m) {
   const lgh_q4 *w[2] = {w1, w3};
   const GemmPlan plan = plan_q4_gemm(w, 2, m);

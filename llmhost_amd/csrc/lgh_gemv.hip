@@ -1281,7 +1281,7 @@ Q4BatchPlan plan_q4_batch(size_t m, size_t bpr) {
   return p;
 }
 
-// Rows of more than 64 blocks (two or four K slices per row group) are
+// Rows of more than 64 blocks (2, 4 or 8 K slices per row group) are
 // quantized once by act_quant_kernel: inside the kernel every workgroup would
 // quantize all m rows, m * k elements (256 workgroups at K=8192, N=2048).
 // Measured, whole call: K=8192, N=2048, M=2 / 4 9.47 / 10.05 -> 7.35 /
@@ -1410,7 +1410,8 @@ hipError_t launch_q4_gemv_mma(const lgh_q4 *const *w, float *const *y, int nmat,
 }
 
 // The gate/up launch keeps q4_mma_kernel's sums, so it stands in for plans of one
-// or two token tiles in 8-block chunks over 8 K slices (33 to 192 blocks a row).
+// or two token tiles in 8-block chunks over 8 K slices: rows of 33 blocks and more,
+// with one token tile up to 192 (from 185 on the general path's kernel loads ahead).
 bool q4_mma_glu_wanted(const lgh_q4 *w1, size_t m) {
   const Q4MmaPlan p = plan_q4_mma(w1->n, m, w1->bpr);
   return p.ok && p.TT <= 2 && p.KW == 8 && p.CB == 8 && w1->n % 32 == 0 && (p.TT == 2 || w1->bpr <= 192);

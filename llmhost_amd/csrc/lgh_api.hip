@@ -986,11 +986,11 @@ static int materialize(lgh_ctx *ctx, const ActIn &in, size_t m, size_t k, const 
 // activation quantization of each route (the MMA image, the GEMM's operand
 // image) is done once and read by every matrix.  m == 1 quantizes inside its
 // kernel, per matrix; 2 <= m <= 4 once for all matrices, rows of up to 64 blocks
-// inside the kernel (with the norm).  The rows may be rms_norm(x) or
-// silu(x) * u (ActIn): the MMA and GEMM routes form them in the launch that
-// writes their activation image (the normed rows are never written), the
-// others, where they do not norm in the kernel, after one more launch that
-// writes them out.
+// inside the kernel (with the norm where q4_batch_norms).  The rows may be
+// rms_norm(x) or silu(x) * u (ActIn): the MMA and GEMM routes form them in the
+// launch that writes their activation image (the normed rows are never
+// written), the others, where they do not norm in the kernel, after one more
+// launch that writes them out.
 static int gemm_multi_dev(lgh_ctx *ctx, const Ws &wsp, const lgh_q4 *const *w, int nmat, ActIn in,
                           float *const *y_dev, size_t m, int mode) {
   const size_t k = w[0]->k, bpr = w[0]->bpr;
@@ -1023,7 +1023,7 @@ static int gemm_multi_dev(lgh_ctx *ctx, const Ws &wsp, const lgh_q4 *const *w, i
           return e;
       return hipSuccess;
     };
-    if (!in.u && lgh::q4_batch_norms(bpr) && !norms_in_place(w, nmat, in.x, in.nw, y_dev, m)) {
+    if (in.nw && lgh::q4_batch_norms(w, nmat) && !norms_in_place(w, nmat, in.x, in.nw, y_dev, m)) {
       // The rows normed and quantized inside the kernel.
       LGH_HIP(ctx, batch(in.x, nullptr, nullptr, in.nw, ctx->act_mode));
       return LGH_OK;

@@ -483,7 +483,7 @@ hipError_t launch_batch(Q4BatchArgs a, hipStream_t st) {
       return hipGetLastError();
     }
   }
-  if (a.nw) return hipErrorInvalidValue;  // q4_batch_norms
+  if (a.nw) return hipErrorInvalidValue;  // rows of <= 64 blocks only
   hipLaunchKernelGGL((q4_gemv_batch_kernel<4, BPL, KW, W, PREQ, false>), grid, blk, 0, st, a);
   return hipGetLastError();
 }
@@ -1289,7 +1289,19 @@ Q4BatchPlan plan_q4_batch(size_t m, size_t bpr) {
 // 8.25 / 8.90 -> 8.04 / 8.37 us.
 bool q4_batch_quantize_once(size_t bpr) { return bpr > 64; }
 
-bool q4_batch_norms(size_t bpr) { return bpr <= 64; }
+// The norm in the kernel saves a launch, but every workgroup norms the rows, in
+// each round of workgroups on a CU.  So up to one workgroup a CU, and up to two
+// over rows of 32 blocks and more.  Norm and one matrix, M = 2, a launch of its
+// own against the kernel: N=8192 (256 workgroups), K=256 / 2048 5.4 / 8.7 -> 5.0 / 7.0
+// us; N=16384, K=256 / 512 6.2 / 6.6 against 6.6 / 7.0 us, K=1024 / 2048 8.0 / 11.1 ->
+// 7.9 / 10.3 us; N=20480, K=256 / 2048 6.7 / 12.6 against 8.3 / 12.9 us; N=32768,
+// K=256 / 2048 7.4 / 14.9 against 10.1 / 16.5 us; two matrices of these rows alike.
+bool q4_batch_norms(const lgh_q4 *const *w, int nmat) {
+  const size_t bpr = w[0]->bpr;
+  size_t wgs = 0;
+  for (int j = 0; j < nmat; j++) wgs += (w[j]->n + 31) / 32;
+  return bpr <= 64 && wgs <= (bpr >= 32 ? 512 : 256);
+}
 
 hipError_t launch_q4_gemv_batch(const lgh_q4 *const *w, float *const *y, int nmat, const float *x,
                                 const int8_t *codes, const float *scales, const float *norm_w, float eps, size_t m,

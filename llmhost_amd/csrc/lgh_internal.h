@@ -198,9 +198,10 @@ Q4BatchPlan plan_q4_batch(size_t m, size_t bpr);
 // reads the codes: inside it, every workgroup would quantize all m rows.
 bool q4_batch_quantize_once(size_t bpr);
 // codes / scales (ActQ8 of the m rows, [m][k] and [m][k/32]) replace x when
-// non-null.  Up to three matrices with the same k in one launch; norm_w (not
-// null only where q4_batch_norms): rms_norm of the rows in the prologue.
-bool q4_batch_norms(size_t bpr);
+// non-null.  Up to three matrices with the same k in one launch; norm_w (rows
+// of <= 64 blocks only): rms_norm of the rows in the prologue.
+// q4_batch_norms: whether a call takes that rather than rms_norm before.
+bool q4_batch_norms(const lgh_q4 *const *w, int nmat);
 hipError_t launch_q4_gemv_batch(const lgh_q4 *const *w, float *const *y, int nmat, const float *x,
                                 const int8_t *codes, const float *scales, const float *norm_w, float eps, size_t m,
                                 int mode, int per_row, hipStream_t st);

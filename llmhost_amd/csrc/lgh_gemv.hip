@@ -1423,10 +1423,18 @@ hipError_t launch_q4_gemv_mma(const lgh_q4 *const *w, float *const *y, int nmat,
 
 // The gate/up launch keeps q4_mma_kernel's sums, so it stands in for plans of one
 // or two token tiles in 8-block chunks over 8 K slices: rows of 33 blocks and more,
-// with one token tile up to 192 (from 185 on the general path's kernel loads ahead).
+// with one token tile up to 192.  Below 192 workgroups (6144 rows of h) a wave's
+// chain of chunks, twice the separate launches', counts: there only up to 184
+// blocks a row (one tile; longer ones load ahead in q4_mma_kernel) or 144 (two).
+// The block, separate launches against this one: M = 24, dim 4608 / 5120 / 6144 /
+// 8192, inter 2048 33.2 / 33.8 / 35.4 / 40.1 against 33.0 / 34.7 / 37.5 / 43.8 us, inter 6144
+// 49.5 / 51.7 / 57.1 / 66.4 -> 42.0 / 43.6 / 46.7 / 53.3 us; M = 13, dim 6144, inter 2048 /
+// 6144 28.4 / 43.8 against 29.1 / 36.0 us.
 bool q4_mma_glu_wanted(const lgh_q4 *w1, size_t m) {
   const Q4MmaPlan p = plan_q4_mma(w1->n, m, w1->bpr);
-  return p.ok && p.TT <= 2 && p.KW == 8 && p.CB == 8 && w1->n % 32 == 0 && (p.TT == 2 || w1->bpr <= 192);
+  const size_t few = p.TT == 1 ? 184 : 144, most = p.TT == 1 ? 192 : SIZE_MAX;
+  return p.ok && p.TT <= 2 && p.KW == 8 && p.CB == 8 && w1->n % 32 == 0 &&
+         w1->bpr <= (w1->n < 6144 ? few : most);
 }
 
 hipError_t launch_q4_mma_glu(const lgh_q4 *w1, const lgh_q4 *w3, const uint8_t *codes, const float *scales, size_t m,

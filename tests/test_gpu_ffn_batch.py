@@ -2,8 +2,8 @@
 bit: every token slot count, rows that end inside a block group, a down projection whose kernel
 takes codes (inter 2080-8192), f32 rows (shorter) or the matrix-core batch route (longer); from 5
 tokens on, one and two token tiles, block counts of h that pad its image's quad by 0 to 3, rows of
-33 to 65 blocks and one more slice chunk, of 192 (the longest that one token tile fuses), 193 and 257;
-both act-quant modes, with and without the norm."""
+33 to 65 blocks and one more slice chunk, and on both sides of the longest that are fused; both act-quant
+modes, with and without the norm."""
 
 import numpy as np
 import pytest
@@ -19,7 +19,7 @@ pytestmark = pytest.mark.gpu
                                               (1056, 64, 4), (2048, 10752, 3), (1536, 8224, 4),
                                               (1536, 8192, 13), (1056, 128, 5), (2048, 160, 16), (2080, 192, 17),
                                               (1568, 2272, 32), (4128, 256, 9),
-                                              (6144, 160, 9), (6176, 160, 9), (6176, 160, 20), (8224, 128, 32)])
+                                              (5888, 160, 9), (5920, 160, 9), (4608, 160, 20), (4640, 160, 20)])
 def test_ffn_few_tokens_equals_op_sequence(gpu_ctx, dim, inter, tokens, norm, per_row):
     shapes = ((inter, dim), (inter, dim), (dim, inter))
     w1, w3, w2 = (q4.Q4Matrix.from_blocks(n, k, synth.q4_blocks(50 + i + n, n, k), gpu_ctx)
@@ -45,6 +45,12 @@ def test_ffn_few_tokens_equals_op_sequence(gpu_ctx, dim, inter, tokens, norm, pe
         for w in (w1, w3, w2):
             w.free()
     assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("dim,inter,tokens", [(6144, 6144, 9), (6176, 6144, 20)])
+def test_ffn_few_tokens_long_rows(gpu_ctx, dim, inter, tokens):
+    """Blocks of enough rows that the gate/up launch takes their longer rows too."""
+    test_ffn_few_tokens_equals_op_sequence(gpu_ctx, dim, inter, tokens, True, False)
 
 
 @pytest.mark.parametrize("warm,captured", [("PerBlock", "PerRow"), ("PerRow", "PerBlock")])

@@ -846,12 +846,18 @@ hipError_t launch_q4_gemm(const lgh_q4 *const *w, int nmat, const uint8_t *mxa, 
 // Without split K or K groups: those add an element's parts in another f32
 // order, and the block's results stay the general path's bits.  That leaves
 // launches of >= 512 128 x 32 tiles of the general path (256 workgroups here),
-// where it won at every size measured (figures above GluCfg), and rows of one
-// block pair (K <= 64), which have no K groups, at any number of tiles.
+// where it won at every size measured (figures above GluCfg) but one: at 256
+// workgroups, one wave a SIMD, rows of 64 block pairs and more, which the general
+// path's two waves a SIMD walk faster.  The block, general path against this one,
+// M = 97, dim 2048 / 4096 / 6144 / 8192: inter 8192 (256 workgroups) 41.9 / 59.4 / 79.1 /
+// 96.4 against 40.1 / 60.0 / 81.8 / 101.7 us; inter 9216 (288) 46.5 / 68.4 / 92.1 / 114.3 ->
+// 44.1 / 65.9 / 89.2 / 112.5 us.  Rows of one block pair (K <= 64), which have no K
+// groups, take it at any number of tiles.
 bool q4_glu_wanted(const lgh_q4 *w1, const lgh_q4 *w3, size_t m) {
   const lgh_q4 *w[2] = {w1, w3};
   const GemmPlan plan = plan_q4_gemm(w, 2, m);
-  return plan.splits == 1 && plan.kgroups == 1 && w1->pp > 0;
+  const size_t wgs = (w1->nt + 1) / 2 * (((m + 31) / 32 + 1) / 2);
+  return plan.splits == 1 && plan.kgroups == 1 && w1->pp > 0 && (w1->pp < 64 || wgs > 256);
 }
 
 hipError_t launch_q4_glu(const lgh_q4 *w1, const lgh_q4 *w3, const uint8_t *mxa, size_t m, uint8_t *img,

@@ -37,3 +37,9 @@ def test_ffn_glu_equals_op_sequence(gpu_ctx, dim, inter, tokens, big, norm):
     for w in (w1, w3, w2):
         w.free()
     assert np.array_equal(got, ref, equal_nan=True)
+
+
+def test_ffn_glu_long_rows(gpu_ctx):
+    """Both sides of the rule for rows of 64 block pairs and more: 256 workgroups and more."""
+    for dim, inter in ((4032, 8192), (4064, 8192), (4096, 8224)):
+        test_ffn_glu_equals_op_sequence(gpu_ctx, dim, inter, 100, False, True)

@@ -28,6 +28,8 @@
 // other half go before the next load asks for it); a K slice per wave with the
 // activations in registers 37 us; two or four chunks in flight 24.8-28.5 us;
 // without the limit to 128 registers 41 / 47 us at 48 / 64 tokens (34 / 39).
+#include <algorithm>
+
 #include "lgh_device.h"
 #include "lgh_internal.h"
 
@@ -253,14 +255,22 @@ hipError_t launch_tt(const Q8MmaArgs &a, hipStream_t st) {
 // row per token costs its share of the stream each.  So the bytes that the pass
 // saves have to be worth the chain: measured crossings at K=1024, N=32003
 // (35 MB) between 2 and 3 tokens (13.4 against 13.0 us, 18.7 against 13), at
-// K=1536, N=65536 below 2 (30.9 against 24.0 us), at K=2048, N=8192 (18 MB) at 5
-// (16 against 14 us at 6).  Fewer rows leave most CUs without a workgroup.  Rows
-// longer than one launch of the GEMV covers stay with its K ranges, whose sums
-// are closer to the 64-bit result there.
+// K=1536, N=65536 below 2 (30.9 against 24.0 us), at K=2048, N=12000 (26 MB)
+// between 4 and 5 (17.5 against 17.9 us, 21.5).  Where the GEMV has a multiple of 8
+// workgroups a token (of 8 waves: N < 12288, a multiple of 256), all tokens'
+// workgroups of a row group run on one XCD and find its share of a matrix of up
+// to 18 MiB in its L2, so that a token costs about half: crossings at N=8192, K=512 /
+// 1024 / 1536 / 2048 at 16 / 13 / 9 / 7 tokens (8.2 / 10.6 / 14.0 / 17.2 us), where
+// N=8456 has them at 10 / 7 / 6 / 6.  Fewer rows leave most CUs without a workgroup.
+// Rows longer than one launch of the GEMV covers stay with its K ranges, whose
+// sums are closer to the 64-bit result there.
 bool q8_batch_wanted(const lgh_q8 *w, size_t tokens) {
-  const size_t chunks = (w->bpr + kChunk - 1) / kChunk;
-  return tokens >= 2 && w->bpr > 0 && w->k <= kQ8GemvMaxK && w->n >= 8192 &&
-         (tokens - 1) * (w->n * w->bpr * 34) >= ((size_t{32} + 8 * chunks) << 20);
+  if (tokens < 2 || w->bpr == 0 || w->k > kQ8GemvMaxK || w->n < 8192) return false;
+  const size_t chunks = (w->bpr + kChunk - 1) / kChunk, bytes = w->n * w->bpr * 34;
+  const Q4GemvPlan p = plan_q4_gemv(w->n, w->bpr, 1, false);
+  const bool in_l2 = p.W == 8 && p.wgs_per_mat % 8 == 0 && bytes <= (size_t{18} << 20);
+  const size_t chain = in_l2 ? std::min(32 + 16 * chunks, 96 + 2 * chunks) : 32 + 8 * chunks;
+  return (tokens - 1) * bytes >= chain << 20;
 }
 
 hipError_t launch_q8_mma(const lgh_q8 *w, const uint8_t *codes, const float *scales, float *y, size_t m,

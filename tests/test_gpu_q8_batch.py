@@ -80,6 +80,20 @@ def test_q8_batch_is_as_exact_as_one_token(gpu_ctx, oracle, k, tokens):
     assert err[0] <= 1.05 * err[1]
 
 
+@pytest.mark.parametrize("n,k", [(8192, 512), (8192, 1024), (9216, 1536), (8448, 2048), (8456, 1024), (12288, 512)])
+def test_q8_batch_rule(gpu_ctx, oracle, n, k):
+    """On both sides of the rule that chooses between the pass and a GEMV row per token."""
+    blocks = synth.q8_blocks(n + k, n, k)
+    w = q4.Q8Matrix.from_blocks(n, k, blocks, gpu_ctx)
+    x = synth.activations(5, 24, k)
+    ref = oracle.q8_apply(blocks, n, k, x, 24, threads=8).reshape(24, n)
+    for tokens in (2, 6, 7, 8, 9, 12, 13, 17, 20, 24):
+        y = np.zeros((tokens, n), dtype=np.float32)
+        q4.q8_apply(w, x[:tokens].copy(), tokens, y)
+        assert_close(y, ref[:tokens], what=f"q8 {n}x{k} m={tokens}")
+    w.free()
+
+
 def test_q8_rows_past_one_launch_take_the_token_route(gpu_ctx):
     """K ranges of 32768 elements: several tokens equal one at a time, bit for bit."""
     n, k, tokens = 8192, 32800, 2

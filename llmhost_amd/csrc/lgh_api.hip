@@ -116,7 +116,8 @@ void trim_stage(lgh_ctx *ctx) {
 // Beyond 512 KB the copies themselves dominate (M=32: 102 us either way), and the
 // pageable path stays; a call that finds the buffer taken by another thread's
 // uses it too.  The buffer is made by the first call that wants it and freed
-// with the last context.
+// with the last context; coherent memory by name, as host and kernels write it in
+// turn and the default can be set by the environment (the times are the same).
 constexpr size_t kPinBytes = size_t(512) << 10;  // each way
 std::mutex g_pin_mu;        // held for a whole call
 char *g_pin = nullptr;      // guarded by g_pin_mu
@@ -132,7 +133,8 @@ struct PinLease {
     if (!lock) return;
     if (!g_pin) {
       void *p = nullptr;
-      if (hipHostMalloc(&p, 2 * kPinBytes, hipHostMallocPortable) != hipSuccess) {
+      if (hipHostMalloc(&p, 2 * kPinBytes, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) !=
+          hipSuccess) {
         (void)hipGetLastError();
         return;
       }

@@ -100,7 +100,8 @@ int lgh_sync(lgh_ctx *ctx);
  * later call grows one of them, lgh_trim or lgh_destroy; and as graphs and
  * eager calls of one context write the same workspaces, the caller orders them
  * (one stream, or events between streams).  Neither holds for Q8_0 calls, which
- * use none when captured (lgh_q8_gemv).  No reference
+ * use none when captured (lgh_q8_gemv; but lgh_q8_norm_gemv's normed rows of
+ * more than 32768 elements).  No reference
  * counterpart (llm-cpu keeps no device buffers). */
 int lgh_trim(lgh_ctx *ctx);
 
@@ -265,7 +266,7 @@ int lgh_probe_read_dev(lgh_ctx *ctx, const void *src_dev, size_t bytes, int per_
  * K ranges of 32768, added in f32).  Several tokens of a large matrix share
  * one pass over the weights per 64 tokens, on an activation image: eager calls
  * share one of the context, a captured call gets one of its own from the matrix,
- * so that its graph needs the matrix, x and y only -- it may be replayed on any
+ * so that its graph needs the matrix and its operands only -- it may be replayed on any
  * stream, beside other calls, and after lgh_destroy.  A matrix holds the images
  * of captured calls until lgh_q8_free, up to 64 MiB; a call past that, as one
  * without device memory for its image, reads the weights once per token.  The
